@@ -364,6 +364,14 @@ int swl_rmsnorm_rows_bf16(void* h, int64_t ntok, int64_t d, const void* const* a
 int swl_silu_mul_rows_bf16(const void* const* in_rows, void* const* out_rows, int64_t ntok, int64_t inter,
                            void* stream);
 
+/* The same two operations over contiguous rows, any number of them in one
+ * launch: out [n, d] = LlamaRMSNorm of x [n, d] (worker_sync.py:314-319,
+ * :1344-1350); out [n, inter] = silu(gate) * up of gu [n, 2 * inter], gate
+ * columns first (worker_sync.py:158).  Bit for bit the row forms.  d and
+ * inter multiples of 8, pointers 16-byte aligned. */
+int swl_rmsnorm_bf16(const void* x, const void* weight, float eps, void* out, int64_t n, int64_t d, void* stream);
+int swl_silu_mul_bf16(const void* gu, void* out, int64_t n, int64_t inter, void* stream);
+
 /* swl_paged_attention_bf16 with per-token rows: token t = seq * q_len + i
  * reads its fused [q | k | v] row at qkv_rows[t] (RoPE applied in place) and
  * writes its [hq * d] output row at out_rows[t].  rope = 2: q in the rows is

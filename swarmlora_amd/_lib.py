@@ -121,6 +121,8 @@ _SIGS = {
                                   ctypes.POINTER(c_int)]),
     "swl_rmsnorm_rows_bf16": (c_int, [c_vp, c_i64, c_i64, P_vp, c_vp, c_f32, P_vp, c_vp]),
     "swl_silu_mul_rows_bf16": (c_int, [P_vp, P_vp, c_i64, c_i64, c_vp]),
+    "swl_rmsnorm_bf16": (c_int, [c_vp, c_vp, c_f32, c_vp, c_i64, c_i64, c_vp]),
+    "swl_silu_mul_bf16": (c_int, [c_vp, c_vp, c_i64, c_i64, c_vp]),
     "swl_paged_attention_rows_bf16": (c_int, [P_vp, P_vp, c_int, c_int, c_int, c_int, c_int, c_vp, c_vp, c_i64,
                                               c_int, c_vp, c_i64, c_vp, c_vp, c_vp, c_i64, c_int, c_f32, c_vp]),
 }

@@ -2840,22 +2840,79 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(bf16* __restrict__ h,
   }
 }
 
-// out[t][j] = bf16(bf16(silu(g)) * u), g = in[t][j], u = in[t][inter + j]
-// (F.silu(gate) * up in bf16, worker_sync.py:158, :1397).
-__global__ __launch_bounds__(256) void silu_mul_rows_kernel(RowPtrs r, int64_t inter) {
-  const int t = blockIdx.y;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (inter >> 3)) return;
+// One 16-byte piece of SiLU(gate) * up: bf16(bf16(silu(g)) * u)
+__device__ __forceinline__ u32x4 silu_mul8(u32x4 gate, u32x4 up) {
   float g[8], u[8];
-  unpack8(ld16(r.in[t] + 8 * i), g);
-  unpack8(ld16(r.in[t] + inter + 8 * i), u);
+  unpack8(gate, g);
+  unpack8(up, u);
   bf16x8 o;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float sg = bf2f(f2bf(g[j] / (1.0f + __expf(-g[j]))));
     o[j] = f2bf(sg * u[j]);
   }
-  *reinterpret_cast<u32x4*>(r.out[t] + 8 * i) = __builtin_bit_cast(u32x4, o);
+  return __builtin_bit_cast(u32x4, o);
+}
+
+// out[t][j] = bf16(bf16(silu(g)) * u), g = in[t][j], u = in[t][inter + j]
+// (F.silu(gate) * up in bf16, worker_sync.py:158, :1397).
+__global__ __launch_bounds__(256) void silu_mul_rows_kernel(RowPtrs r, int64_t inter) {
+  const int t = blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (inter >> 3)) return;
+  *reinterpret_cast<u32x4*>(r.out[t] + 8 * i) = silu_mul8(ld16(r.in[t] + 8 * i), ld16(r.in[t] + inter + 8 * i));
+}
+
+// Dense forms of the two row kernels for a worker's prompt chunk: x [n, d]
+// contiguous, any number of rows in one launch (the row forms take 64 rows of
+// pointers a launch: 512 rows of both were 16 launches of 3-4 us each).
+// Memory bound: each input row is read once and kept in registers (up to
+// kNormVec 16-byte pieces a thread, d <= 8192), where the row form reads it
+// twice.  The sums run in the row form's order, so both give the same bits.
+// 512 rows of 4096 and of 2 x 14336, both calls in turn, host included:
+// 142 us in 64-row launches, 15 us in one each.
+constexpr int kNormVec = 4;
+__global__ __launch_bounds__(256) void rmsnorm_dense_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                            bf16* __restrict__ out, int64_t d, float eps) {
+  __shared__ float sh[4];
+  const bf16* xr = x + (int64_t)blockIdx.x * d;
+  bf16* yr = out + (int64_t)blockIdx.x * d;
+  const int64_t nv = d >> 3;
+  u32x4 q[kNormVec];
+#pragma unroll
+  for (int i = 0; i < kNormVec; ++i) {
+    const int64_t v = threadIdx.x + 256 * i;
+    q[i] = v < nv ? ldg16(xr + 8 * v) : u32x4{0u, 0u, 0u, 0u};
+  }
+  float ss = 0.f;
+  auto add = [&](u32x4 p) {
+    float f[8];
+    unpack8(p, f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += f[j] * f[j];
+  };
+#pragma unroll
+  for (int i = 0; i < kNormVec; ++i) add(q[i]);  // pieces past the row add zeros
+  for (int64_t v = threadIdx.x + 256 * kNormVec; v < nv; v += 256) add(ldg16(xr + 8 * v));
+  ss = block_reduce<float>(ss, [](float a, float b) { return a + b; }, sh);
+  const float rs = rsqrtf(ss / (float)d + eps);
+#pragma unroll
+  for (int i = 0; i < kNormVec; ++i) {
+    const int64_t v = threadIdx.x + 256 * i;
+    if (v < nv) *reinterpret_cast<u32x4*>(yr + 8 * v) = norm8(q[i], rs, ldg16(w + 8 * v));
+  }
+  for (int64_t v = threadIdx.x + 256 * kNormVec; v < nv; v += 256)
+    *reinterpret_cast<u32x4*>(yr + 8 * v) = norm8(ldg16(xr + 8 * v), rs, ldg16(w + 8 * v));
+}
+
+__global__ __launch_bounds__(256) void silu_mul_dense_kernel(const bf16* __restrict__ gu, bf16* __restrict__ out,
+                                                             int64_t n, int64_t inter) {
+  const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (v >= (inter >> 3)) return;
+  for (int64_t t = blockIdx.y; t < n; t += gridDim.y) {
+    const bf16* r = gu + t * 2 * inter + 8 * v;
+    *reinterpret_cast<u32x4*>(out + t * inter + 8 * v) = silu_mul8(ldg16(r), ldg16(r + inter));
+  }
 }
 
 // ------------------------------------------------------ embed / LM head ---
@@ -5097,6 +5154,31 @@ extern "C" int swl_rmsnorm_rows_bf16(void* h, int64_t ntok, int64_t d, const voi
   hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)ntok), dim3(256), 0, (hipStream_t)stream,
                      reinterpret_cast<bf16*>(h), d, r, reinterpret_cast<const bf16*>(weight), eps, add_rows ? 1 : 0);
   SWL_LAUNCH_CHECK("rmsnorm_rows_kernel launch");
+  return SWL_OK;
+}
+
+extern "C" int swl_rmsnorm_bf16(const void* x, const void* weight, float eps, void* out, int64_t n, int64_t d,
+                                void* stream) {
+  SWL_CHECK(n >= 0 && n < ((int64_t)1 << 31), SWL_ERR_INVALID, "swl_rmsnorm_bf16: bad row count");
+  SWL_CHECK(d > 0 && d % 8 == 0, SWL_ERR_INVALID, "swl_rmsnorm_bf16: d must be a multiple of 8");
+  if (n == 0) return SWL_OK;
+  SWL_CHECK(x && weight && out, SWL_ERR_INVALID, "swl_rmsnorm_bf16: null argument");
+  hipLaunchKernelGGL(rmsnorm_dense_kernel, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream,
+                     reinterpret_cast<const bf16*>(x), reinterpret_cast<const bf16*>(weight),
+                     reinterpret_cast<bf16*>(out), d, eps);
+  SWL_LAUNCH_CHECK("rmsnorm_dense_kernel launch");
+  return SWL_OK;
+}
+
+extern "C" int swl_silu_mul_bf16(const void* gu, void* out, int64_t n, int64_t inter, void* stream) {
+  SWL_CHECK(n >= 0, SWL_ERR_INVALID, "swl_silu_mul_bf16: bad row count");
+  SWL_CHECK(inter > 0 && inter % 8 == 0, SWL_ERR_INVALID, "swl_silu_mul_bf16: inter must be a multiple of 8");
+  if (n == 0) return SWL_OK;
+  SWL_CHECK(gu && out, SWL_ERR_INVALID, "swl_silu_mul_bf16: null argument");
+  const dim3 grid((unsigned)(((inter >> 3) + 255) / 256), (unsigned)std::min<int64_t>(n, 65535));
+  hipLaunchKernelGGL(silu_mul_dense_kernel, grid, dim3(256), 0, (hipStream_t)stream,
+                     reinterpret_cast<const bf16*>(gu), reinterpret_cast<bf16*>(out), n, inter);
+  SWL_LAUNCH_CHECK("silu_mul_dense_kernel launch");
   return SWL_OK;
 }
 

@@ -211,3 +211,35 @@ def test_engine_silu_mul_reads_fused_halves(dev, t, inter):
     assert bits_equal(a, b)
     want = ref.silu_mul(gu[..., :inter].cpu(), gu[..., inter:].cpu())
     assert_close(a.cpu(), want, what="engine silu*up")
+
+
+@pytest.mark.parametrize("n,d", [(1, 8), (65, 2056), (513, 4096), (3, 8192), (2, 8200), (2, 20488)])
+def test_dense_norm_and_act_match_row_forms(dev, n, d):
+    """The one-launch norm and SiLU*up over n contiguous rows (rows held in
+    registers up to d = 8192, re-read past it) against the row forms, bit for
+    bit, one launch of at most 64 rows at a time."""
+    ops = _ops()
+    x, gu = randn((n, d), 21).to(dev), randn((n, 2 * d), 22, std=2.0).to(dev)
+    w = (1 + randn((d,), 23, std=0.1).float()).to(BF16).to(dev)
+    norm, act = ops.rms_norm(x, w, 1e-5), ops.silu_mul(gu, d)
+    want_n, want_a = torch.zeros_like(x), torch.zeros_like(x)
+    for c in range(0, n, 64):
+        rows = list(range(c, min(n, c + 64)))
+        ops.rmsnorm_rows(x[c:c + 64].clone(), w, 1e-5, [want_n[t] for t in rows])
+        ops.silu_mul_rows([gu[t] for t in rows], [want_a[t] for t in rows], d)
+    torch.cuda.synchronize()
+    assert bits_equal(norm, want_n) and bits_equal(act, want_a)
+
+
+def test_dense_act_more_rows_than_the_grid(dev):
+    """70000 rows of 8 columns: rows past the grid's second dimension."""
+    ops = _ops()
+    gu = randn((70000, 16), 24, std=2.0).to(dev)
+    got = ops.silu_mul(gu, 8)
+    torch.cuda.synchronize()
+    for c in (0, 65535, 69999):
+        want = torch.zeros(8, dtype=BF16, device=dev)
+        ops.silu_mul_rows([gu[c]], [want], 8)
+        torch.cuda.synchronize()
+        assert bits_equal(got[c], want)
+    assert ops.rms_norm(gu[:0], torch.ones(16, dtype=BF16, device=dev), 1e-5).shape == (0, 16)
