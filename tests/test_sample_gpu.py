@@ -125,3 +125,71 @@ def test_embed_rows_bit_exact_with_clamped_ids(dev, vocab, hidden):
         assert bits_equal(o[: w.shape[0]].cpu(), w), f"slot {i}"
     # an empty slot's buffer is not written
     assert bool((outs[2] == 7.0).all())
+
+
+def _expected_draw(row, T, k, p, seed, r):
+    """The sampler's rule for one row in float64 on the CPU: keep the k
+    largest scaled values (ties kept), of those the sorted prefix whose mass
+    is within p (the most likely token always), then the first index whose
+    cumulative kept mass passes u * mass.  Returns (token, the set of tokens
+    next to it that a target within 1e-6 of a boundary could give)."""
+    def mix(x):
+        m = (1 << 64) - 1
+        for c in (0xff51afd7ed558ccd, 0xc4ceb9fe1a85ec53):
+            x ^= x >> 33
+            x = x * c & m
+        return x ^ (x >> 33)
+
+    inv = (torch.ones(1) / torch.tensor([T], dtype=torch.float32))[0]
+    v = (row.float() * inv).double()
+    e = (v - v.max()).exp()
+    kept = torch.ones_like(v, dtype=torch.bool)
+    if 0 < k < v.numel():
+        kept = v >= v.topk(k).values[-1]
+    if p < 1.0:
+        vals, inverse = torch.unique(v[kept], return_inverse=True)  # ascending
+        mass = torch.zeros_like(vals).index_add_(0, inverse, e[kept])
+        tail = mass.flip(0).cumsum(0).flip(0)                       # mass of values >= each
+        ok = tail <= float(torch.tensor(p, dtype=torch.float32)) * tail[0]
+        kept &= (v >= vals[ok][0]) if bool(ok.any()) else torch.zeros_like(kept)
+    kept[row.float().argmax()] = True
+    cdf = torch.where(kept, e, torch.zeros_like(e)).cumsum(0)
+    u = (mix((seed * 0x9e3779b97f4a7c15 + r + 1) % (1 << 64)) >> 40) / (1 << 24)
+    pick = [int((cdf <= (u + d) * cdf[-1]).sum()) for d in (-1e-6, 0.0, 1e-6)]
+    return pick[1], set(pick)
+
+
+@pytest.mark.parametrize("vocab,std", [(128256, 2.0), (128256, 0.01), (5000, 3.0), (1001, 2.0), (517, 40.0), (9, 1.0),
+                                       (300000, 2.0), (2200000, 2.0)])
+@pytest.mark.parametrize("k,p", [(0, 1.0), (50, 1.0), (0, 0.9), (50, 0.9), (1000, 0.3), (3, 0.0), (0, 0.999)])
+def test_draw_follows_the_rule(dev, vocab, std, k, p):
+    """Every threshold combination against the rule in float64: rows aligned
+    and not, vocabularies under and over what one group per block covers,
+    values spread over many bins or squeezed into one, -inf and tied rows."""
+    g = torch.Generator().manual_seed(vocab + k)
+    n = 6 if vocab < 1000000 else 2
+    lg = (torch.randn(n, vocab, generator=g) * std).to(torch.bfloat16)
+    lg[0, ::2] = -math.inf
+    if n > 2:
+        lg[2] = 1.5  # all tied
+    T = 0.8
+    got = _run(lg.to(dev), True, temperature=T, top_k=k, top_p=p, seed=21).tolist()
+    for r in range(n):
+        _, near = _expected_draw(lg[r], T, k, p, 21, r)
+        assert got[r] in near, (r, got[r], near)
+
+
+def test_draw_with_nan_or_inf_is_the_largest(dev):
+    """A NaN, or an infinite logit (whose probability against itself is a
+    NaN), in the kept set leaves no distribution: the argmax is taken; one
+    that top-k drops does not matter."""
+    lg = torch.randn(4, 1000, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    lg[0, 7], lg[1, 8], lg[2, 9] = math.nan, math.inf, -math.nan
+    lg[3, :] = -math.inf
+    neg_nan = torch.tensor([-64], dtype=torch.int16).view(torch.bfloat16)[0]  # 0xffc0: below every value
+    lg[2, 9] = neg_nan
+    got = _run(lg.to(dev), True, temperature=0.9, seed=2).tolist()
+    top = lg[2].float().nan_to_num(nan=-math.inf).argmax().item()
+    assert got == [7, 8, top, 0]
+    kept = _run(lg.to(dev), True, temperature=0.9, top_k=5, seed=2).tolist()
+    assert kept[2] in lg[2].float().nan_to_num(nan=-math.inf).topk(5).indices.tolist()
