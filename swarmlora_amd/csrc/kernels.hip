@@ -30,7 +30,8 @@
 //   matmul_generic_kernel   small row-major products with arbitrary strides
 //                           (worker-side LoRA modules).
 //   rope_append_kernel, attn_tile_kernel + attn_combine_kernel (decode),
-//   attn_chunk_kernel, attention_kernel     paged-KV attention.
+//   attn_chunk_kernel (decode), attn_prefill_kernel (q_len > 1)
+//                           paged-KV attention.
 //
 // MFMA used: v_mfma_f32_16x16x32_bf16 (decode rounds, attention, shrink) and
 // v_mfma_f32_32x32x16_bf16 (gemm256_kernel).  16x16x32 operand layout
@@ -2131,137 +2132,458 @@ __device__ __forceinline__ bf16* tok_out(const AttnArgs& a, int64_t t) {
 }
 
 // NeoX rotation of q and k at their positions, k/v appended to the pages.
-// One 64-thread workgroup per (token, head) of the fused row: q heads are
-// rotated in place, k heads rotated in place and copied to the K page, v
-// heads copied to the V page (lane d handles dims d and d + 64).
-__global__ __launch_bounds__(64) void rope_append_kernel(AttnArgs a) {
-  const int tokid = blockIdx.x;  // s * L + i
-  const int h = blockIdx.y;      // [0, hq): q, [hq, hq + hkv): k, then v
-  const int d = threadIdx.x;
-  const int s = tokid / a.L, i = tokid % a.L;
+// A 128-thread workgroup per (token, 16 heads), eight threads a head with
+// 16-byte accesses: thread c takes dims 8 c .. + 7 and the same of the other
+// half.  q heads are rotated in place, k heads rotated in place and copied to
+// the K page, v heads copied to the V page.  The position's factors and the
+// page are requested along with the row: the kernel is a chain of latencies
+// for a few tokens, and short of bytes in flight for many (512 tokens of 32 +
+// 16 heads: 9.4 us with a 64-thread workgroup per head and 2-byte accesses,
+// @ROPE@ now; 28 tokens: 3.5, @ROPE28@).
+__global__ __launch_bounds__(128) void rope_append_kernel(AttnArgs a) {
+  const int64_t tokid = blockIdx.x;                     // s * L + i
+  const int h = blockIdx.y * 16 + (threadIdx.x >> 3);   // [0, hq): q, [hq, hq + hkv): k, then v
+  if (h >= a.hq + 2 * a.hkv) return;
+  const int d = 8 * (threadIdx.x & 7);
+  const int64_t s = a.L == 1 ? tokid : tokid / a.L, i = tokid - s * a.L;
   const bool is_q = h < a.hq, is_k = !is_q && h < a.hq + a.hkv;
-  bf16* row = is_q ? tok_q(a, tokid) + h * 128
-                   : (is_k ? tok_k(a, tokid) + (h - a.hq) * 128
-                           : const_cast<bf16*>(tok_v(a, tokid)) + (h - a.hq - a.hkv) * 128);
-  float x1 = bf2f(row[d]), x2 = bf2f(row[d + 64]);
-  if (!is_q && !is_k) {
-    // v: copy only
-  } else if (a.rope) {
-    const int64_t pos = a.pos[tokid];
-    if (pos >= 0 && pos < a.max_pos) {
-      const bf16* cs = a.cs + pos * 128;
-      const float c = bf2f(cs[d]), sn = bf2f(cs[64 + d]);
-      const float y1 = x1 * c - x2 * sn, y2 = x2 * c + x1 * sn;
-      const bf16 o1 = f2bf(y1), o2 = f2bf(y2);
-      row[d] = o1;
-      row[d + 64] = o2;
-      x1 = bf2f(o1);
-      x2 = bf2f(o2);
-    }
-  }
-  if (is_q) return;
+  bf16* row = (is_q ? tok_q(a, tokid) + h * 128
+                    : (is_k ? tok_k(a, tokid) + (h - a.hq) * 128
+                            : const_cast<bf16*>(tok_v(a, tokid)) + (h - a.hq - a.hkv) * 128)) + d;
+  u32x4 w1 = ldg16(row), w2 = ldg16(row + 64);
+  const int64_t pos = a.rope ? a.pos[tokid] : -1;
   const int64_t p = (int64_t)a.seqlens[s] + i;
-  const int64_t blk_i = p / a.bs;
-  if (p < 0 || blk_i >= a.max_blocks) return;
-  const int32_t blk = a.bt[(int64_t)s * a.max_blocks + blk_i];
-  if (blk < 0 || blk >= a.num_blocks) return;
-  const int kvh = is_k ? h - a.hq : h - a.hq - a.hkv;
-  bf16* dst = (is_k ? a.kc : a.vc) + ((int64_t)blk * a.bs + p % a.bs) * a.hkv * 128 + kvh * 128;
-  dst[d] = f2bf(x1);
-  dst[d + 64] = f2bf(x2);
-}
-
-// Attention of one query token over its causal context for one kv head and
-// its G = hq / hkv query heads.  Workgroup = 4 waves; each 16-lane quarter of
-// a wave owns one key at a time (lane holds 8 of the 128 dims), so a wave
-// consumes 4 keys per step and the workgroup 16 keys (one page) per step.
-// Online softmax per quarter; quarters are merged through LDS at the end.
-template <int G>
-__global__ __launch_bounds__(256) void attention_kernel(AttnArgs a) {
-  const int h = blockIdx.x;       // kv head
-  const int i = blockIdx.y;       // query index within the group
-  const int s = blockIdx.z;       // sequence
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int quarter = tid >> 4;   // 0..15 across the workgroup
-  const int dl = (lane & 15) * 8; // this lane's 8 dims
-  const int64_t ctx = (int64_t)a.seqlens[s] + i + 1;
-
-  float qv[G][8];
+  const int64_t blk_i = a.bs_shift >= 0 ? p >> a.bs_shift : p / a.bs;
+  const int32_t blk = p >= 0 && blk_i < a.max_blocks ? a.bt[s * a.max_blocks + blk_i] : -1;
+  if ((is_q || is_k) && pos >= 0 && pos < a.max_pos) {
+    const bf16* cs = a.cs + pos * 128 + d;
+    float x1[8], x2[8], c[8], sn[8];
+    if ((reinterpret_cast<uintptr_t>(a.cs) & 15) == 0) {
+      unpack8(ldg16(cs), c);
+      unpack8(ldg16(cs + 64), sn);
+    } else {
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const bf16* qp = tok_q(a, (int64_t)s * a.L + i) + (h * G + g) * 128 + dl;
-    unpack8(ld16(qp), qv[g]);
-#pragma unroll
-    for (int d = 0; d < 8; ++d) qv[g][d] *= a.scale;
-  }
-  float mx[G], sm[G], acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    mx[g] = -INFINITY;
-    sm[g] = 0.f;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) acc[g][d] = 0.f;
-  }
-  const int32_t* bt = a.bt + (int64_t)s * a.max_blocks;
-  const int64_t rowstride = (int64_t)a.hkv * 128;
-  for (int64_t key = quarter; key < ctx; key += 16) {
-    const int64_t bi = key / a.bs;
-    int32_t blk = (bi < a.max_blocks) ? bt[bi] : -1;
-    if (blk < 0 || blk >= a.num_blocks) continue;
-    const int64_t off = ((int64_t)blk * a.bs + key % a.bs) * rowstride + h * 128 + dl;
-    float kv[8], vv[8];
-    unpack8(ld16(a.kc + off), kv);
-    unpack8(ld16(a.vc + off), vv);
-    float sc[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float t = 0.f;
-#pragma unroll
-      for (int d = 0; d < 8; ++d) t += qv[g][d] * kv[d];
-      sc[g] = t;
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-      for (int o = 8; o >= 1; o >>= 1) sc[g] += __shfl_xor(sc[g], o, 16);
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float nm = fmaxf(mx[g], sc[g]);
-      const float corr = __expf(mx[g] - nm);
-      const float p = __expf(sc[g] - nm);
-      sm[g] = sm[g] * corr + p;
-#pragma unroll
-      for (int d = 0; d < 8; ++d) acc[g][d] = acc[g][d] * corr + p * vv[d];
-      mx[g] = nm;
-    }
-  }
-  // merge the 16 quarters
-  __shared__ float smx[16][G], ssm[16][G];
-  __shared__ float sacc[16][G][128];
-  if ((lane & 15) == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) { smx[quarter][g] = mx[g]; ssm[quarter][g] = sm[g]; }
-  }
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int d = 0; d < 8; ++d) sacc[quarter][g][dl + d] = acc[g][d];
-  __syncthreads();
-  for (int it = tid; it < G * 128; it += 256) {
-    const int g = it >> 7, d = it & 127;
-    float m = -INFINITY;
-    for (int qq = 0; qq < 16; ++qq) m = fmaxf(m, smx[qq][g]);
-    float l = 0.f, o = 0.f;
-    if (m != -INFINITY) {
-      for (int qq = 0; qq < 16; ++qq) {
-        const float c = (smx[qq][g] == -INFINITY) ? 0.f : __expf(smx[qq][g] - m);
-        l += ssm[qq][g] * c;
-        o += sacc[qq][g][d] * c;
+      for (int e = 0; e < 8; ++e) {
+        c[e] = bf2f(cs[e]);
+        sn[e] = bf2f(cs[64 + e]);
       }
     }
-    const float r = (l > 0.f) ? o / l : 0.f;
-    tok_out(a, (int64_t)s * a.L + i)[(h * G + g) * 128 + d] = f2bf(r);
+    unpack8(w1, x1);
+    unpack8(w2, x2);
+    bf16x8 o1, o2;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      o1[e] = f2bf(x1[e] * c[e] - x2[e] * sn[e]);
+      o2[e] = f2bf(x2[e] * c[e] + x1[e] * sn[e]);
+    }
+    w1 = __builtin_bit_cast(u32x4, o1);
+    w2 = __builtin_bit_cast(u32x4, o2);
+    *reinterpret_cast<u32x4*>(row) = w1;
+    *reinterpret_cast<u32x4*>(row + 64) = w2;
+  }
+  if (is_q || blk < 0 || blk >= a.num_blocks) return;
+  const int kvh = is_k ? h - a.hq : h - a.hq - a.hkv;
+  bf16* dst = (is_k ? a.kc : a.vc) + ((int64_t)blk * a.bs + (p - blk_i * a.bs)) * a.hkv * 128 + kvh * 128 + d;
+  *reinterpret_cast<u32x4*>(dst) = w1;
+  *reinterpret_cast<u32x4*>(dst + 64) = w2;
+}
+
+// ---- attention of q_len > 1 tokens (prompt chunks) ----------------------
+// One workgroup per (kv head, block of 32 rows, sequence), a row being one
+// query head of one new token (row = token * G + head, so the G heads sharing
+// a kv head share its K and V).  Wave w of KH takes the steps of 32 keys w,
+// w + KH, ... on its own: no barrier until the waves' results of each row are
+// merged in LDS at the end (no scratch memory and no second launch, so calls
+// on several streams stay independent).
+//
+// S^T = K . Q^T and O^T = V^T . P^T on 16x16x32 MFMA: a lane holds keys
+// 4 g .. + 3 (g = lane / 16) of each 16-key tile of one row, which is the B
+// operand of the second product as it is when MFMA k-group g is taken as keys
+// 4 g .. + 3 of both tiles.  K rows are loaded as MFMA operands; V goes
+// through the wave's LDS as key quads ([quad][dim] x 4 keys, transposed in
+// registers on the way in).  The next step's K and V are requested as soon as
+// the current ones leave their registers.  The probabilities enter as the sum
+// of two bf16 (the rounded value and what the rounding left, 2^-17 of it
+// unaccounted), two products per tile: the result differs from fp32
+// probabilities by far less than its own rounding (measured against 64 bits:
+// 2.5e-3 before and after).
+//
+// What bounded the kernel this replaces was vector work: one query token per
+// workgroup, every K and V row read again for each.  What bounds this one is
+// the CU's load path: clock stamps show a step's 16 KB of K and V taking
+// 1000-3000 cycles to issue and arrive against ~2700 of its own work (128 KB
+// per round of 8 waves, about 25 bytes a cycle).  Staging 64 rows' K and V
+// through LDS with two barriers a tile was level (31 us); the reads of V four
+// tiles ahead of their products and the two row sets' maxima together: ctx
+// 512, 512 tokens, 33.7 against 38.5 us a pass.  512 tokens over 1024 keys,
+// 32 / 8 heads, under the trace: 320 -> 32 us.
+constexpr int kPaVQuad = 1152;                    // bytes of a key quad's 128 dims x 4 keys, 128 of skew
+constexpr int kPaVBytes = 8 * kPaVQuad;           // V of a wave's 32 keys
+constexpr int kPaMerge = 68 * 64 * 4;             // a wave's partial result: 68 floats a lane
+constexpr int pa_lds_bytes(int kh) {              // V of every wave, then half the waves' results; a flag per wave
+  return (kh * kPaVBytes > kh / 2 * kPaMerge ? kh * kPaVBytes : kh / 2 * kPaMerge) + kh * 4;
+}
+
+// One row by one wave on vector arithmetic, seeing only its own keys: 16
+// lanes a key (8 dims each), 4 keys a step, the four quarters merged last.
+__device__ __forceinline__ void attn_row(const AttnArgs& a, int s, int h, int gsh, int r, int lane) {
+  const int64_t t = (int64_t)s * a.L + (r >> gsh);
+  const int64_t off = (int64_t)((h << gsh) + (r & ((1 << gsh) - 1))) * 128 + 8 * (lane & 15);
+  const int64_t end = min<int64_t>((int64_t)a.seqlens[s] + (r >> gsh) + 1, a.max_blocks * a.bs);
+  const int32_t* bt = a.bt + (int64_t)s * a.max_blocks;
+  float q[8], acc[8], mx = -INFINITY, sm = 0.f;
+  unpack8(ldg16(tok_q(a, t) + off), q);
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    q[d] *= a.scale;
+    acc[d] = 0.f;
+  }
+  for (int64_t key = lane >> 4; key < end; key += 4) {
+    const int64_t bi = key / a.bs;
+    const int32_t pb = bt[bi];
+    if (pb < 0 || pb >= a.num_blocks) continue;
+    const int64_t at = (((int64_t)pb * a.bs + (key - bi * a.bs)) * a.hkv + h) * 128 + 8 * (lane & 15);
+    float kf[8], vf[8], sc = 0.f;
+    unpack8(ldg16(a.kc + at), kf);
+    unpack8(ldg16(a.vc + at), vf);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) sc += q[d] * kf[d];
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) sc += __shfl_xor(sc, o, 16);
+    const float nm = fmaxf(mx, sc), corr = __expf(mx - nm), p = __expf(sc - nm);
+    sm = sm * corr + p;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[d] = acc[d] * corr + p * vf[d];
+    mx = nm;
+  }
+  for (int o = 16; o <= 32; o += 16) {
+    const float mo = __shfl_xor(mx, o, 64), so = __shfl_xor(sm, o, 64), nm = fmaxf(mx, mo);
+    const float ca = mx == -INFINITY ? 0.f : __expf(mx - nm), cb = mo == -INFINITY ? 0.f : __expf(mo - nm);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[d] = acc[d] * ca + __shfl_xor(acc[d], o, 64) * cb;
+    sm = sm * ca + so * cb;
+    mx = nm;
+  }
+  if (lane < 16) {
+    bf16x8 o;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[d] = f2bf(sm > 0.f ? acc[d] / sm : 0.f);
+    bf16* dst = tok_out(a, t) + off;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) stg(dst + d, o[d]);
+  }
+}
+  // bytes of a key quad's 128 dims x 4 keys, 128 of skew
+// P16: pages are whole 16-key tiles (one cache offset per tile, found 64 tiles
+// at a time); else the offset of every key is looked up.
+template <int KH, bool P16>
+__global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, int gsh) {
+  extern __shared__ __attribute__((aligned(16))) char pa_lds[];
+  uint32_t* vbad = reinterpret_cast<uint32_t*>(pa_lds + pa_lds_bytes(KH) - KH * 4);
+  const int lane = threadIdx.x & 63;
+  const int kh = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int h = blockIdx.x, s = blockIdx.z;
+  const int blk = gridDim.y - 1 - blockIdx.y;  // the blocks with the most keys first
+  const int rows = a.L << gsh, r0 = blk * 32;
+  const int64_t len = a.seqlens[s];
+  const int64_t ctx_lo = len + (r0 >> gsh) + 1;                           // of the block's first row
+  const int64_t ctx_hi = len + ((min(r0 + 32, rows) - 1) >> gsh) + 1;     // of its last
+  const int64_t kend = min<int64_t>(ctx_hi, a.max_blocks * a.bs);          // no page past the table
+  const int nsteps = kend > 32 * kh ? (int)((kend - 32 * kh + 32 * KH - 1) / (32 * KH)) : 0;
+  const int64_t krow = (int64_t)a.hkv * 128;
+  const int32_t* bt = a.bt + (int64_t)s * a.max_blocks;
+
+  // the block's rows (set e: 16 of them, this lane's is column l % 16) as the
+  // B operand, and the context of this lane's row of each set
+  u32x4 qf[2][4];
+  int64_t ctx[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int r = min(r0 + e * 16 + col, rows - 1);
+    const bf16* qp = tok_q(a, (int64_t)s * a.L + (r >> gsh)) + (int64_t)((h << gsh) + (r & ((1 << gsh) - 1))) * 128;
+#pragma unroll
+    for (int st = 0; st < 4; ++st) qf[e][st] = ldg16(qp + 32 * st + 8 * g);
+    ctx[e] = len + (r >> gsh) + 1;
+  }
+
+  // cache offset (elements) of the key, -1: past the context, or no page
+  auto offset_of = [&](int64_t key) {
+    if (key >= kend) return (int64_t)-1;
+    const int64_t bi = a.bs_shift >= 0 ? key >> a.bs_shift : key / a.bs;
+    const int32_t pb = bt[bi];
+    return pb >= 0 && pb < a.num_blocks ? ((int64_t)pb * a.bs + (key - bi * a.bs)) * krow : (int64_t)-1;
+  };
+  // P16: lane 2 i + t holds the offset of tile t of step j0 + i (a table of
+  // 32 steps); else lane t holds that of key t of the step loaded last
+  int64_t table = -1;
+  auto look = [&](int j) {
+    if constexpr (P16) {
+      if ((j & 31) == 0) table = offset_of(((int64_t)(j + (lane >> 1)) * KH + kh) * 32 + 16 * (lane & 1));
+    } else {
+      table = offset_of(((int64_t)j * KH + kh) * 32 + (lane & 31));
+    }
+  };
+  auto from_lane = [&](int l) {
+    return (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)(table & 0xffffffff), l) |
+           ((int64_t)__builtin_amdgcn_readlane((int)(table >> 32), l) << 32);
+  };
+  const bf16* kc = a.kc + h * 128;
+  const bf16* vc = a.vc + h * 128;
+  // bit k of none: no key k in the step (of those that `look` found)
+  u32x4 kr[2][4], vr[2][4];
+  uint32_t none_next = 0;
+  auto load_k = [&](int j) {
+    look(j);
+    none_next = 0;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const bf16* kp;
+      if constexpr (P16) {
+        const int64_t b = from_lane(2 * (j & 31) + kt);
+        none_next |= b < 0 ? 0xffffu << (16 * kt) : 0u;
+        kp = kc + (b < 0 ? 0 : b) + ((uint32_t)col * (uint32_t)krow + 8 * g);
+      } else {
+        const int64_t b = __shfl((long long)table, 16 * kt + col, 64);
+        kp = kc + (b < 0 ? 0 : b) + 8 * g;
+      }
+#pragma unroll
+      for (int st = 0; st < 4; ++st) kr[kt][st] = ldg16(kp + 32 * st);
+    }
+    if constexpr (!P16) none_next = (uint32_t)__ballot(table < 0);
+  };
+  // V: items n: keys 16 n + 4 g .. + 3, dims 8 (l % 16) .. + 7
+  auto load_v = [&](int j) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      if constexpr (P16) {
+        const int64_t b = from_lane(2 * (j & 31) + n);
+        const bf16* vp = vc + (b < 0 ? 0 : b) + ((uint32_t)(4 * g) * (uint32_t)krow + 8 * col);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) vr[n][q] = ldg16(vp + q * krow);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int64_t b = __shfl((long long)table, 16 * n + 4 * g + q, 64);
+          vr[n][q] = ldg16(vc + (b < 0 ? 0 : b) + 8 * col);
+        }
+      }
+    }
+  };
+  char* vlds = pa_lds + kh * kPaVBytes;
+
+  // scores in powers of two; the kernel takes a positive factor, a negative
+  // one's sign goes to the products (scale 0: all scores 0)
+  const float cs2 = a.scale * 1.44269504088896340736f;
+  const float c2 = cs2 == 0.f ? 1.f : fabsf(cs2);
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+  f32x4 acc[2][8];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[e][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t nonfinite = 0;  // V of a step that some rows see part of holds an infinity or NaN
+
+  if (nsteps > 0) {
+    load_k(0);
+    load_v(0);
+  }
+  for (int j = 0; j < nsteps; ++j) {
+    const int64_t k0 = ((int64_t)j * KH + kh) * 32;
+    const uint32_t none = none_next;
+    // a row of the block ends inside the step, or a key is missing
+    const bool edge = k0 + 32 > ctx_lo;
+    f32x4 sv[2][2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      sv[kt][0] = sv[kt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        sv[kt][0] = mfma16(kr[kt][st], qf[0][st], sv[kt][0]);
+        sv[kt][1] = mfma16(kr[kt][st], qf[1][st], sv[kt][1]);
+      }
+    }
+    if (j + 1 < nsteps) load_k(j + 1);
+
+    // V of this step into LDS, rows without a key as zeros (their
+    // probability is 0, what the page holds there is anything)
+    if (edge || none) {
+      const int live = (int)min<int64_t>(32, kend - k0);
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int k = 16 * n + 4 * g + q;
+          if (k >= live || (none >> k & 1)) vr[n][q] = u32x4{0u, 0u, 0u, 0u};
+          if (edge) {
+            uint32_t bad = 0;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+              const uint32_t w = vr[n][q][p];
+              bad |= ((w & 0x7f80u) == 0x7f80u || (w & 0x7f800000u) == 0x7f800000u) ? 1u : 0u;
+            }
+            nonfinite |= bad;
+          }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      char* dst = vlds + (4 * n + g) * kPaVQuad + col * 64;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const uint32_t w0 = vr[n][0][p], w1 = vr[n][1][p], w2 = vr[n][2][p], w3 = vr[n][3][p];
+        *reinterpret_cast<u32x4*>(dst + ((p ^ (col >> 2)) << 4)) =
+            u32x4{__builtin_amdgcn_perm(w1, w0, 0x05040100u), __builtin_amdgcn_perm(w3, w2, 0x05040100u),
+                  __builtin_amdgcn_perm(w1, w0, 0x07060302u), __builtin_amdgcn_perm(w3, w2, 0x07060302u)};
+      }
+    }
+    if (j + 1 < nsteps) load_v(j + 1);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    if (!(cs2 > 0.f))
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) sv[kt][e] = cs2 == 0.f ? f32x4{0.f, 0.f, 0.f, 0.f} : -sv[kt][e];
+    if (edge || none) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int see = (int)min<int64_t>(32, ctx[e] - k0);  // keys of the 32 that this lane's row sees
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int k = 16 * kt + 4 * g + q;
+            if (k >= see || (none >> k & 1)) sv[kt][e][q] = -INFINITY;
+          }
+      }
+    }
+    // V operands, four tiles of 16 dims ahead of their products
+    const char* vp = vlds + g * kPaVQuad + (col >> 3) * 64 + (col & 1) * 8;
+    auto v_at = [&](int d) {
+      const char* vd = vp + d * 128 + ((((col & 7) >> 1) ^ (d >> 1)) << 4);
+      const u32x2 v0 = *reinterpret_cast<const u32x2*>(vd);
+      const u32x2 v1 = *reinterpret_cast<const u32x2*>(vd + 4 * kPaVQuad);
+      return u32x4{v0[0], v0[1], v1[0], v1[1]};
+    };
+    u32x4 vf[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) vf[d] = v_at(d);
+
+    float mx[2] = {-INFINITY, -INFINITY};
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) mx[e] = fmaxf(mx[e], sv[q >> 2][e][q & 3]);
+#pragma unroll
+    for (int o = 16; o <= 32; o += 16)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) mx[e] = fmaxf(mx[e], __shfl_xor(mx[e], o, 64));
+    // the reference the exponents are taken from moves only when a maximum
+    // has grown by 2^8 since: any reference gives the same quotient, and the
+    // sums are far from overflow
+    if (__ballot(mx[0] * c2 > m[0] + 8.f || mx[1] * c2 > m[1] + 8.f) != 0) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float mn = fmaxf(m[e], mx[e] * c2);
+        const float corr = mn == m[e] ? 1.f : __builtin_amdgcn_exp2f(m[e] - mn);
+        m[e] = mn;
+        l[e] *= corr;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) acc[e][d] *= corr;
+      }
+    }
+    u32x4 ph[2], pl[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float mr = m[e] == -INFINITY ? 0.f : m[e];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {  // keys in pairs: one conversion for both
+        const f32x4& x = sv[q >> 1][e];
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(x[2 * (q & 1)], c2, -mr));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(x[2 * (q & 1) + 1], c2, -mr));
+        l[e] += p0;
+        l[e] += p1;
+        const uint32_t hi = __builtin_bit_cast(uint32_t, (bf16x2){f2bf(p0), f2bf(p1)});
+        ph[e][q] = hi;
+        pl[e][q] = __builtin_bit_cast(uint32_t, (bf16x2){f2bf(p0 - __uint_as_float(hi << 16)),
+                                                         f2bf(p1 - __uint_as_float(hi & 0xffff0000u))});
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) acc[e][d] = mfma16(vf[d & 3], ph[e], acc[e][d]);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) acc[e][d] = mfma16(vf[d & 3], pl[e], acc[e][d]);
+      if (d < 4) vf[d] = v_at(d + 4);
+    }
+    __builtin_amdgcn_wave_barrier();  // (LDS accesses of a wave stay in order: the reads precede the next writes)
+  }
+
+  if (lane == 0) vbad[kh] = 0;
+  if (__ballot(nonfinite != 0) != 0 && lane == 0) vbad[kh] = 1;
+  __syncthreads();
+  uint32_t again = 0;
+#pragma unroll
+  for (int w = 0; w < KH; ++w) again |= vbad[w];
+  if (again) {  // uniform over the workgroup
+    // such a value's key has probability 0 in a row that does not see it, and
+    // 0 times it is a NaN: these rows again, key by key
+    for (int r = r0 + kh; r < min(r0 + 32, rows); r += KH) attn_row(a, s, h, gsh, r, lane);
+    return;
+  }
+
+  // the row sums over the four lane groups, then the KH waves of a row merged
+  // pairwise through LDS (each lane meets the same lane of the other wave)
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    l[e] += __shfl_xor(l[e], 16, 64);
+    l[e] += __shfl_xor(l[e], 32, 64);
+  }
+  for (int half = KH / 2; half >= 1; half >>= 1) {
+    if (half < KH / 2) __syncthreads();
+    float* mg = reinterpret_cast<float*>(pa_lds) + (int64_t)(kh % half) * 68 * 64;
+    if (kh >= half && kh < 2 * half) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+#pragma unroll
+        for (int d = 0; d < 8; ++d) *reinterpret_cast<f32x4*>(mg + ((e * 8 + d) * 64 + lane) * 4) = acc[e][d];
+        mg[(64 + 2 * e) * 64 + lane] = m[e];
+        mg[(65 + 2 * e) * 64 + lane] = l[e];
+      }
+    }
+    __syncthreads();
+    if (kh < half) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float mo = mg[(64 + 2 * e) * 64 + lane], lo = mg[(65 + 2 * e) * 64 + lane];
+        const float mn = fmaxf(m[e], mo);
+        const float ca = mn == m[e] ? 1.f : __builtin_amdgcn_exp2f(m[e] - mn);
+        const float cb = mn == mo ? 1.f : __builtin_amdgcn_exp2f(mo - mn);
+        m[e] = mn;
+        l[e] = l[e] * ca + lo * cb;
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+          acc[e][d] = acc[e][d] * ca + *reinterpret_cast<const f32x4*>(mg + ((e * 8 + d) * 64 + lane) * 4) * cb;
+      }
+    }
+  }
+  if (kh != 0) return;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int r = r0 + e * 16 + col;
+    if (r >= rows) continue;
+    bf16* op = tok_out(a, (int64_t)s * a.L + (r >> gsh)) + (int64_t)((h << gsh) + (r & ((1 << gsh) - 1))) * 128;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = l[e] > 0.f ? acc[e][d][q] / l[e] : 0.f;
+      store4_bf16(v, 16 * d + 4 * g, 128, op);
+    }
   }
 }
 
@@ -4151,10 +4473,35 @@ bool attn_tile_fits(const AttnArgs& a) {
   return attn_tile_tuning().on && a.L == 1 && a.bs % kTileKeys == 0;
 }
 
+template <int KH, bool P16>
+int launch_attn_prefill_t(const AttnArgs& a, int gsh, hipStream_t st) {
+  static size_t allowed = 0;
+  constexpr size_t lds = pa_lds_bytes(KH);
+  int rc = allow_lds(attn_prefill_kernel<KH, P16>, lds, &allowed);
+  if (rc) return rc;
+  const int64_t blocks = (((int64_t)a.L << gsh) + 31) / 32;
+  hipLaunchKernelGGL((attn_prefill_kernel<KH, P16>), dim3((unsigned)a.hkv, (unsigned)blocks, (unsigned)a.nseq),
+                     dim3(64 * KH), lds, st, a, gsh);
+  SWL_LAUNCH_CHECK("attn_prefill_kernel launch");
+  return SWL_OK;
+}
+
+// Waves a workgroup (its keys are dealt over them): 8 while the blocks of 32
+// rows do not outnumber the CUs (the registers leave a CU 8 waves), 4 past
+// that.  Cache offsets per 16-key tile where pages are whole tiles.
+int launch_attn_prefill(const AttnArgs& a, int G, hipStream_t st) {
+  const int gsh = __builtin_ctz((unsigned)G);
+  const int64_t blocks = (((int64_t)a.L << gsh) + 31) / 32 * a.hkv * a.nseq;
+  const bool p16 = a.bs % 16 == 0;
+  if (blocks <= cu_count())
+    return p16 ? launch_attn_prefill_t<8, true>(a, gsh, st) : launch_attn_prefill_t<8, false>(a, gsh, st);
+  return p16 ? launch_attn_prefill_t<4, true>(a, gsh, st) : launch_attn_prefill_t<4, false>(a, gsh, st);
+}
+
 int launch_attention(const AttnArgs& a, int G, hipStream_t st) {
   if (a.rope <= 1) {  // 2: q rotated and k / v appended by the QKV round's epilogue
-    hipLaunchKernelGGL(rope_append_kernel, dim3((unsigned)(a.nseq * a.L), (unsigned)(a.hq + 2 * a.hkv)), dim3(64),
-                       0, st, a);
+    hipLaunchKernelGGL(rope_append_kernel, dim3((unsigned)(a.nseq * a.L), (unsigned)((a.hq + 2 * a.hkv + 15) / 16)),
+                       dim3(128), 0, st, a);
     SWL_LAUNCH_CHECK("rope_append_kernel launch");
   }
   if (a.L == 1 && attn_tile_fits(a)) {
@@ -4173,15 +4520,7 @@ int launch_attention(const AttnArgs& a, int G, hipStream_t st) {
       default: return launch_attn_decode_u<8>(a, st);
     }
   }
-  const dim3 grid((unsigned)a.hkv, (unsigned)a.L, (unsigned)a.nseq);
-  switch (G) {
-    case 1: hipLaunchKernelGGL(attention_kernel<1>, grid, dim3(256), 0, st, a); break;
-    case 2: hipLaunchKernelGGL(attention_kernel<2>, grid, dim3(256), 0, st, a); break;
-    case 4: hipLaunchKernelGGL(attention_kernel<4>, grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL(attention_kernel<8>, grid, dim3(256), 0, st, a); break;
-  }
-  SWL_LAUNCH_CHECK("attention_kernel launch");
-  return SWL_OK;
+  return launch_attn_prefill(a, G, st);
 }
 
 }  // namespace

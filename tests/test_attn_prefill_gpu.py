@@ -1,0 +1,132 @@
+"""GPU tests of attention over several new tokens per sequence (prompt
+chunks): block and tile edges of the MFMA kernel, pages of any size, missing
+pages, and infinite or NaN values that causality hides from some rows.
+
+The reference is the definition in float64 on the CPU.  Bound per element:
+the result's rounding to bf16 (2^-9 of its size, itself at most the largest
+|V|), the fp32 accumulation over the context and the probabilities' 2^-17:
+4e-3 of the largest |V| covers them.
+"""
+
+import math
+
+import pytest
+import torch
+
+from tests._util import BF16, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(dev, nseq, L, hq, hkv, ctx, page, missing=()):
+    """Random q/k/v over shuffled pages (no RoPE); `missing`: (sequence, page
+    index) entries of the block table set to -1."""
+    per = (max(ctx) + L + page - 1) // page + 1
+    nb = nseq * per
+    c = {"q": randn((nseq, L, hq, 128), 1), "k": randn((nseq, L, hkv, 128), 2), "v": randn((nseq, L, hkv, 128), 3),
+         "kc": randn((nb, page, hkv, 128), 4), "vc": randn((nb, page, hkv, 128), 5),
+         "bt": torch.randperm(nb, generator=torch.Generator().manual_seed(6)).reshape(nseq, per).to(torch.int32),
+         "len": torch.tensor(ctx, dtype=torch.int32)}
+    for s, j in missing:
+        c["bt"][s, j] = -1
+    return c
+
+
+def _run(dev, c, scale):
+    from swarmlora_amd import ops
+    d = {k: v.to(dev) for k, v in c.items()}
+    out = ops.paged_attention(d["q"], d["k"], d["v"], d["kc"], d["vc"], d["bt"], d["len"], None, None, scale, rope=False)
+    torch.cuda.synchronize()
+    return out.cpu().double(), d
+
+
+def _want(c, scale):
+    nseq, L, hq, _ = c["q"].shape
+    hkv, page = c["k"].shape[2], c["kc"].shape[1]
+    kc, vc = c["kc"].double(), c["vc"].double()
+    out = torch.zeros(nseq, L, hq * 128, dtype=torch.float64)
+    for s in range(nseq):
+        n = int(c["len"][s])
+        for i in range(L):
+            b = int(c["bt"][s, (n + i) // page])
+            if b >= 0:
+                kc[b, (n + i) % page], vc[b, (n + i) % page] = c["k"][s, i].double(), c["v"][s, i].double()
+        keys = torch.arange(n + L)
+        blocks = c["bt"][s][keys // page].long()
+        ks, vs = kc[blocks.clamp_min(0), keys % page], vc[blocks.clamp_min(0), keys % page]
+        for i in range(L):
+            see = (blocks >= 0) & (keys < n + i + 1)
+            if not bool(see.any()):
+                continue
+            for h in range(hq):
+                kv = h * hkv // hq
+                p = ((ks[see][:, kv] @ c["q"][s, i, h].double()) * scale).softmax(0)
+                out[s, i, h * 128:(h + 1) * 128] = p @ vs[see][:, kv]
+    return out
+
+
+def _check(got, want, vmax):
+    bad = ~((got - want).abs() <= 4e-3 * vmax)
+    assert not bool(bad.any()), f"max error {float((got - want).abs().max()):.3e}"
+
+
+# rows per (sequence, kv head) = L * hq / hkv around 32 and 64 (row blocks);
+# contexts around 64, 128 and 256 keys (tiles); more blocks than CUs (the
+# four-wave form) in the last two
+@pytest.mark.parametrize("nseq,L,hq,hkv,ctx,page", [
+    (1, 2, 4, 4, [0], 16), (1, 31, 4, 4, [33], 16), (1, 33, 4, 4, [0], 16), (2, 8, 16, 4, [224, 3], 16),
+    (3, 9, 32, 4, [255, 0, 47], 16), (1, 16, 32, 8, [1000], 16), (2, 65, 8, 2, [63, 129], 32),
+    (1, 130, 16, 8, [127], 8), (1, 40, 8, 4, [300], 7), (1, 300, 32, 8, [212], 16),
+    (3, 130, 32, 16, [11, 90, 64], 48), (2, 200, 64, 32, [5, 130], 16),
+])
+def test_prefill_attention_edges(dev, nseq, L, hq, hkv, ctx, page):
+    c = _case(dev, nseq, L, hq, hkv, ctx, page)
+    got, _ = _run(dev, c, 128 ** -0.5)
+    _check(got, _want(c, 128 ** -0.5), 6.0)
+
+
+@pytest.mark.parametrize("scale", [-0.09, 0.5])
+def test_prefill_attention_missing_pages(dev, scale):
+    """Block table entries of -1 hide their keys (a whole first page, one in
+    the middle, a new token's own page), also with a negative scale."""
+    c = _case(dev, 2, 20, 8, 2, [40, 0], 16, missing=((0, 0), (0, 3), (1, 0)))
+    got, d = _run(dev, c, scale)
+    _check(got, _want(c, scale), 6.0)
+    assert bool((got[1, :16] == 0).all())  # no key at all
+
+
+@pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
+@pytest.mark.parametrize("L,ctx", [(40, 10), (100, 200)])
+def test_prefill_attention_keeps_nonfinite_values_causal(dev, value, L, ctx):
+    """A non-finite value of new token 17 reaches the rows that see it and no
+    other; non-finite cache contents past the context reach none."""
+    c = _case(dev, 1, L, 8, 2, [ctx], 16)
+    clean, _ = _run(dev, {k: v.clone() for k, v in c.items()}, 128 ** -0.5)
+    c["v"][0, 17, 1, 5] = value
+    c["vc"][int(c["bt"][0, -1])] = math.nan   # a page past every context
+    c["kc"][int(c["bt"][0, -1])] = math.nan
+    got, _ = _run(dev, c, 128 ** -0.5)
+    hit = torch.zeros(L, 8, 128, dtype=torch.bool)
+    hit[17:, 4:, 5] = True  # kv head 1 serves query heads 4..7
+    hit = hit.reshape(1, L, -1)
+    assert not bool(got[hit].isfinite().any())
+    # the rest as without it; rows computed key by key round differently
+    assert float((got[~hit] - clean[~hit]).abs().max()) <= 4e-3 * 6.0
+
+
+def test_prefill_attention_under_capture_without_a_first_call(dev):
+    """The kernel takes no scratch: a graph can capture the first call ever
+    made with a shape, and replays give the eager result each time."""
+    from swarmlora_amd import ops
+    c = {k: v.to(dev) for k, v in _case(dev, 1, 24, 8, 2, [100], 16).items()}
+    out = torch.zeros(1, 24, 1024, dtype=BF16, device=dev)
+    args = (c["q"], c["k"], c["v"], c["kc"], c["vc"], c["bt"], c["len"], None, None, 0.1)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ops.paged_attention(*args, rope=False, out=out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ops.paged_attention(*args, rope=False))
+        torch.cuda.synchronize()
