@@ -2139,7 +2139,7 @@ __device__ __forceinline__ bf16* tok_out(const AttnArgs& a, int64_t t) {
 // page are requested along with the row: the kernel is a chain of latencies
 // for a few tokens, and short of bytes in flight for many (512 tokens of 32 +
 // 16 heads: 9.4 us with a 64-thread workgroup per head and 2-byte accesses,
-// @ROPE@ now; 28 tokens: 3.5, @ROPE28@).
+// 5.4 now; a decode pass of 28 tokens level).
 __global__ __launch_bounds__(128) void rope_append_kernel(AttnArgs a) {
   const int64_t tokid = blockIdx.x;                     // s * L + i
   const int h = blockIdx.y * 16 + (threadIdx.x >> 3);   // [0, hq): q, [hq, hq + hkv): k, then v
