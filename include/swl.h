@@ -282,6 +282,22 @@ int swl_lora_rows_bf16(const void* x, int64_t ldx, int64_t m, int64_t k,
                        const int64_t* blk_cols, float alpha, void* y,
                        int64_t ldy, void* stream);
 
+/* The same delta for any number of rows (a prompt chunk), in two launches;
+ * same meaning of x, a, b, blk_cols, alpha and y, the same two bf16 roundings.
+ * nr = nblk * rank, rank a multiple of 8 from 8 to 64; x rows, a, every b and
+ * part 16-byte aligned; a either [k, nr] rows (a_sj = 1, a_sk a multiple of 8)
+ * or [nr, k] rows (a_sk = 1, a_sj a multiple of 8); each b either rows of
+ * columns (b_sc = 1, b_srr and the block's columns multiples of 8) or rows of
+ * ranks (b_srr = 1, b_sc a multiple of 8).  part: n_ks * m * nr floats of
+ * scratch for the n_ks (1..64) K-slices of the shrink, owned by the call
+ * until its kernels have run. */
+int swl_lora_delta_bf16(const void* x, int64_t ldx, int64_t m, int64_t k,
+                        const void* a, int64_t a_sk, int64_t a_sj, int64_t nr,
+                        int nblk, int64_t rank, const void* const* b,
+                        const int64_t* b_srr, const int64_t* b_sc,
+                        const int64_t* blk_cols, float alpha, void* y,
+                        int64_t ldy, void* part, int n_ks, void* stream);
+
 /* Paged-KV attention for one q_len group, replacing
  * WorkerBatchedOps.batch_flash_attention (worker_sync.py:169-205).  Token t
  * (t = seq * q_len + i) has its query heads at q + t*q_stride ([hq, d]), its

@@ -2094,6 +2094,275 @@ __global__ __launch_bounds__(256) void lora_rows_kernel(LoraRowsArgs a) {
   }
 }
 
+// LoRA delta of a worker's prompt chunk (more rows than lora_rows takes) in
+// two launches: lora_shrink_kernel, then lora_expand_mfma_kernel.  As scalar
+// products, one output a thread, a layer's four deltas of 512 rows took 999
+// us; their outputs alone are 44 MB (9 us), and x and the adapter 30 MB.
+//
+// Shrink: part[ks][m][j] = x[m, :] . A(:, j) over K-slice ks, fp32.  One
+// workgroup per (32 rows, K-slice, 64 columns of A): its 8 waves take k-steps
+// of 32 in turn (every load of a step in flight at once), on 16x16x32 MFMA
+// with A's columns as the rows of the product, so that a lane ends with 4
+// consecutive columns; the waves' sums meet in LDS.  A as [j][k] rows is the
+// MFMA operand as it lies in memory; as [k][j] rows (fused_A) a step is
+// transposed through the wave's LDS in quads of 4 k ([quad][j] x 4 k).  What
+// bounds it is the latency of a step's loads, so the K-slices are as many as
+// give every CU a few waves, but no more: the expand reads each slice.
+struct LoraDeltaArgs {
+  const bf16* x;
+  int64_t ldx;
+  int m, K, nr, n_ks;
+  const bf16* a;
+  int64_t a_sk, a_sj;
+  float* part;  // [n_ks][m][nr]
+  int nblk, rank;
+  const bf16* b[kLoraRowsMaxBlk];
+  int64_t srr[kLoraRowsMaxBlk], sc[kLoraRowsMaxBlk];
+  int32_t off[kLoraRowsMaxBlk + 1], tile0[kLoraRowsMaxBlk + 1];  // columns, 64-column tiles before block b
+  float alpha;
+  bf16* y;
+  int64_t ldy;
+};
+constexpr int kLdRows = 32;               // rows of a shrink workgroup
+constexpr int kLdQuad = 64 * 8 + 128;     // bytes of a k-quad's 64 columns, skewed: neighbours in other banks
+
+template <bool KMAJOR>  // A as [k][j] rows
+__global__ __launch_bounds__(512) void lora_shrink_kernel(LoraDeltaArgs a) {
+  constexpr int WAVES = 8;
+  __shared__ __attribute__((aligned(16))) char lds[WAVES * 8 * kLdQuad];  // the transposed steps, then the sums
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int r0 = blockIdx.x * kLdRows, ks = blockIdx.y, j0 = blockIdx.z * 64;
+  const int nj = min(64, a.nr - j0);  // columns of this group
+  const int steps = (a.K + 31) / 32;
+  const int st0 = (int)((int64_t)steps * ks / a.n_ks), st1 = (int)((int64_t)steps * (ks + 1) / a.n_ks);
+  const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+  const bf16* xr[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) xr[e] = a.x + (int64_t)min(r0 + 16 * e + col, a.m - 1) * a.ldx + 8 * g;
+  f32x4 acc[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) acc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  char* mine = lds + wv * 8 * kLdQuad;
+  const int quad = lane >> 3, oct = lane & 7;  // this lane's part of a transposed step
+
+  u32x4 xv[2], av[4];
+  auto load = [&](int st) {
+    const int k = 32 * st + 8 * g;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) xv[e] = k < a.K ? ldg16(xr[e] + 32 * st) : zero;
+    if constexpr (KMAJOR) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int kk = 32 * st + 4 * quad + q;
+        av[q] = kk < a.K && 8 * oct < nj ? ldg16(a.a + (int64_t)kk * a.a_sk + j0 + 8 * oct) : zero;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        av[t] = k < a.K && 16 * t < nj
+                    ? ldg16(a.a + (int64_t)min(j0 + 16 * t + col, a.nr - 1) * a.a_sj + 32 * st + 8 * g)
+                    : zero;
+    }
+  };
+  if (st0 + wv < st1) load(st0 + wv);
+  for (int st = st0 + wv; st < st1; st += WAVES) {
+    const u32x4 x0 = xv[0], x1 = xv[1];
+    u32x4 f[4];
+    if constexpr (KMAJOR) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        *reinterpret_cast<u32x4*>(mine + quad * kLdQuad + oct * 64 + 16 * (p ^ (oct >> 1))) =
+            u32x4{__builtin_amdgcn_perm(av[1][p], av[0][p], 0x05040100u), __builtin_amdgcn_perm(av[3][p], av[2][p], 0x05040100u),
+                  __builtin_amdgcn_perm(av[1][p], av[0][p], 0x07060302u), __builtin_amdgcn_perm(av[3][p], av[2][p], 0x07060302u)};
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        // column 16 t + col: octet 2 t + col / 8 (its pieces permuted by octet / 2 = t), 8 k of group g: quads 2 g, 2 g + 1
+        const char* fp = mine + 2 * g * kLdQuad + (2 * t + (col >> 3)) * 64 + 16 * (((col & 7) >> 1) ^ t) + 8 * (col & 1);
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(fp), hi = *reinterpret_cast<const u32x2*>(fp + kLdQuad);
+        f[t] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) f[t] = av[t];
+    }
+    if (st + WAVES < st1) load(st + WAVES);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (16 * t >= nj) break;  // uniform
+      acc[t][0] = mfma16(f[t], x0, acc[t][0]);
+      acc[t][1] = mfma16(f[t], x1, acc[t][1]);
+    }
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses stay in order)
+  }
+  // the waves' sums, one 16-column tile at a time: [wave][e][lane] f32x4
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
+  static_assert(WAVES * 2 * 64 * 16 <= sizeof(lds), "a tile's sums must fit");
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    if (16 * t >= nj) break;  // uniform
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 2; ++e) red[(wv * 2 + e) * 64 + lane] = acc[t][e];
+    __syncthreads();
+    if (wv < 2) {  // wave e: rows 16 e .. of the 32
+      f32x4 s = red[wv * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) s += red[(w * 2 + wv) * 64 + lane];
+      const int row = r0 + 16 * wv + col, j = j0 + 16 * t + 4 * g;
+      if (row < a.m) {
+        float* dst = a.part + ((int64_t)ks * a.m + row) * a.nr + j;
+        if (j < a.nr) *reinterpret_cast<f32x4*>(dst) = s;  // nr is a multiple of 8
+      }
+    }
+  }
+}
+
+// Expand: y[m, c] = bf16(alpha * sum_rr u[m, b * rank + rr] * B_b(rr, c)), b
+// the block that holds column c, u = bf16 of the summed slices (both roundings
+// as the two bf16 products of the reference).  One workgroup per (16 RT rows,
+// 4 tiles of 64 columns): it sums its rows' u into LDS, each wave keeps a
+// tile's B as MFMA operands in registers and runs over the rows.  The product
+// rows of MFMA tile t are columns 16 (rr / 4) + 4 t + rr % 4, so a lane ends
+// with 16 consecutive columns of a row: two 16-byte stores, and a row's 128
+// bytes from one wave.  Bound by the writes of y.
+constexpr int kLdMaxRank = 64;
+template <int KS, int RT>  // rank <= 32 KS
+__global__ __launch_bounds__(256) void lora_expand_mfma_kernel(LoraDeltaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  constexpr int ROWS = 16 * RT;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int r0 = blockIdx.y * ROWS;
+  const int rows = min(ROWS, a.m - r0);
+  const int ldu = a.nr + 8;  // bf16 row pitch of u: a 16-byte multiple off the banks' period
+  bf16* us = reinterpret_cast<bf16*>(lds);
+  char* tr = lds + ROWS * ldu * 2 + wv * (8 * KS * kLdQuad);  // the wave's transposed tile of B
+
+  const int tile = blockIdx.x * 4 + wv;
+  const bool live = tile < a.tile0[a.nblk];
+  int b = 0;
+  while (b + 1 < a.nblk && tile >= a.tile0[b + 1]) ++b;
+  const int c0 = (tile - a.tile0[b]) * 64;               // first column in the block
+  const int nc = live ? min(64, a.off[b + 1] - a.off[b] - c0) : 0;
+  const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+  // B of the tile: operand row rr of MFMA tile t is column 16 (rr / 4) + 4 t +
+  // rr % 4; requested before u is summed
+  const bf16* bp = a.b[b];
+  const bool rows_of_b = a.sc[b] == 1;  // B(rr, :) contiguous, else B(:, c)
+  u32x4 bv[4 * KS];
+  if (rows_of_b) {
+    // quads of 4 rr x 8 columns: item i = lane + 64 n: quad i / 8, octet i % 8
+#pragma unroll
+    for (int n = 0; n < KS; ++n)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int rr = 4 * ((lane >> 3) + 8 * n) + q, c = 8 * (lane & 7);
+        bv[4 * n + q] = rr < a.rank && c < nc ? ldg16(bp + rr * a.srr[b] + c0 + c) : zero;
+      }
+  } else {
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int c = 16 * (col >> 2) + 4 * t + (col & 3), rr = 32 * k + 8 * g;
+        bv[4 * k + t] = rr < a.rank && c < nc ? ldg16(bp + (int64_t)(c0 + c) * a.sc[b] + rr) : zero;
+      }
+  }
+  // u rows of the workgroup, 4 columns an item
+  const int q4 = a.nr >> 2;
+  for (int i = threadIdx.x; i < ROWS * q4; i += 256) {
+    const int r = i / q4, c = 4 * (i - r * q4);
+    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (r < rows) {
+      const float* p = a.part + (int64_t)(r0 + r) * a.nr + c;
+      const int64_t stride = (int64_t)a.m * a.nr;
+      for (int k0 = 0; k0 < a.n_ks; k0 += 4) {
+        f32x4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          v[k] = k0 + k < a.n_ks ? *reinterpret_cast<const f32x4*>(p + (k0 + k) * stride) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s += v[k];
+      }
+    }
+    u32x2 o;
+    o[0] = __builtin_bit_cast(uint32_t, (bf16x2){f2bf(s[0]), f2bf(s[1])});
+    o[1] = __builtin_bit_cast(uint32_t, (bf16x2){f2bf(s[2]), f2bf(s[3])});
+    *reinterpret_cast<u32x2*>(us + r * ldu + c) = o;
+  }
+  u32x4 f[KS][4];
+  if (rows_of_b) {
+#pragma unroll
+    for (int n = 0; n < KS; ++n) {
+      char* dst = tr + ((lane >> 3) + 8 * n) * kLdQuad + (lane & 7) * 64;
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        *reinterpret_cast<u32x4*>(dst + 16 * p) =
+            u32x4{__builtin_amdgcn_perm(bv[4 * n + 1][p], bv[4 * n][p], 0x05040100u),
+                  __builtin_amdgcn_perm(bv[4 * n + 3][p], bv[4 * n + 2][p], 0x05040100u),
+                  __builtin_amdgcn_perm(bv[4 * n + 1][p], bv[4 * n][p], 0x07060302u),
+                  __builtin_amdgcn_perm(bv[4 * n + 3][p], bv[4 * n + 2][p], 0x07060302u)};
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (rows_of_b) {
+        const int c = 16 * (col >> 2) + 4 * t + (col & 3);
+        const char* fp = tr + (8 * k + 2 * g) * kLdQuad + c * 8;
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(fp), hi = *reinterpret_cast<const u32x2*>(fp + kLdQuad);
+        f[k][t] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      } else {
+        f[k][t] = bv[4 * k + t];
+      }
+    }
+  if (!live) return;
+  const bool vec = ((reinterpret_cast<uintptr_t>(a.y) | (uint64_t)(a.ldy * 2) | (uint64_t)(a.off[b] * 2)) & 15) == 0;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    if (16 * rt >= rows) break;  // uniform
+    f32x4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const int rr = 32 * k + 8 * g;
+      const u32x4 uf = rr < a.rank ? lds16(us + (16 * rt + col) * ldu + b * a.rank + rr) : zero;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t] = mfma16(f[k][t], uf, acc[t]);
+    }
+    // lane: row 16 rt + col, columns 16 g + 4 t + j
+    const int row = 16 * rt + col;
+    if (row >= rows) continue;
+    bf16* yr = a.y + (int64_t)(r0 + row) * a.ldy + a.off[b] + c0 + 16 * g;
+    uint32_t o[8];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      o[2 * t] = __builtin_bit_cast(uint32_t, (bf16x2){f2bf(a.alpha * acc[t][0]), f2bf(a.alpha * acc[t][1])});
+      o[2 * t + 1] = __builtin_bit_cast(uint32_t, (bf16x2){f2bf(a.alpha * acc[t][2]), f2bf(a.alpha * acc[t][3])});
+    }
+    if (vec && 16 * g + 16 <= nc) {
+      *(__attribute__((address_space(1))) u32x4*)(yr) = u32x4{o[0], o[1], o[2], o[3]};
+      *(__attribute__((address_space(1))) u32x4*)(yr + 8) = u32x4{o[4], o[5], o[6], o[7]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (16 * g + i < nc)
+          stg(yr + i, __builtin_bit_cast(bf16, (uint16_t)(i & 1 ? o[i >> 1] >> 16 : o[i >> 1] & 0xffffu)));
+    }
+  }
+}
+
 // ------------------------------------------------------ paged attention ---
 struct AttnArgs {
   bf16* q;               // token t at q + t*qs: [hq, 128]
@@ -4863,6 +5132,82 @@ int swl_lora_rows_bf16(const void* x, int64_t ldx, int64_t m, int64_t k, const v
   else
     hipLaunchKernelGGL(lora_rows_kernel<64>, dim3(grid), dim3(256), 0, st, r);
   SWL_LAUNCH_CHECK("lora_rows_kernel launch");
+  return SWL_OK;
+}
+
+int swl_lora_delta_bf16(const void* x, int64_t ldx, int64_t m, int64_t k, const void* a, int64_t a_sk, int64_t a_sj,
+                        int64_t nr, int nblk, int64_t rank, const void* const* b, const int64_t* b_srr,
+                        const int64_t* b_sc, const int64_t* blk_cols, float alpha, void* y, int64_t ldy, void* part,
+                        int n_ks, void* stream) {
+  SWL_CHECK(x && a && b && b_srr && b_sc && blk_cols && y && part, SWL_ERR_INVALID,
+            "swl_lora_delta_bf16: null argument");
+  SWL_CHECK(m >= 0 && m <= ((int64_t)1 << 20) && k > 0 && k <= ((int64_t)1 << 20) && k % 8 == 0, SWL_ERR_INVALID,
+            "swl_lora_delta_bf16: at most 2^20 rows, k a multiple of 8");
+  SWL_CHECK(rank >= 8 && rank <= kLdMaxRank && rank % 8 == 0 && nblk >= 1 && nblk <= kLoraRowsMaxBlk &&
+                nr == nblk * rank,
+            SWL_ERR_INVALID, "swl_lora_delta_bf16: 1..4 blocks of rank 8..64 (a multiple of 8) columns");
+  SWL_CHECK(n_ks >= 1 && n_ks <= 64, SWL_ERR_INVALID, "swl_lora_delta_bf16: 1..64 K-slices");
+  auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  SWL_CHECK(al(x) && al(a) && al(part) && ldx % 8 == 0 && ldx >= k, SWL_ERR_INVALID,
+            "swl_lora_delta_bf16: x rows, A and part must be 16-byte aligned");
+  const bool kmajor = a_sj == 1;
+  SWL_CHECK(kmajor ? a_sk % 8 == 0 && a_sk >= nr : a_sk == 1 && a_sj % 8 == 0 && a_sj >= k, SWL_ERR_INVALID,
+            "swl_lora_delta_bf16: A must be rows of k or of columns, 16-byte aligned");
+  LoraDeltaArgs r{};
+  r.off[0] = r.tile0[0] = 0;
+  for (int i = 0; i < nblk; ++i) {
+    SWL_CHECK(b[i] && blk_cols[i] > 0 && blk_cols[i] <= ((int64_t)1 << 24), SWL_ERR_INVALID,
+              "swl_lora_delta_bf16: empty block");
+    const bool rows = b_sc[i] == 1;
+    SWL_CHECK(al(b[i]) && (rows ? b_srr[i] % 8 == 0 && b_srr[i] >= blk_cols[i] && blk_cols[i] % 8 == 0
+                                : b_srr[i] == 1 && b_sc[i] % 8 == 0 && b_sc[i] >= rank),
+              SWL_ERR_INVALID, "swl_lora_delta_bf16: B must be 16-byte aligned rows of columns or of ranks");
+    r.b[i] = reinterpret_cast<const bf16*>(b[i]);
+    r.srr[i] = b_srr[i];
+    r.sc[i] = b_sc[i];
+    r.off[i + 1] = r.off[i] + (int)blk_cols[i];
+    r.tile0[i + 1] = r.tile0[i] + (int)((blk_cols[i] + 63) / 64);
+  }
+  SWL_CHECK(ldy >= r.off[nblk], SWL_ERR_INVALID, "swl_lora_delta_bf16: ldy below the output columns");
+  if (m == 0) return SWL_OK;
+  r.x = reinterpret_cast<const bf16*>(x);
+  r.ldx = ldx;
+  r.m = (int)m;
+  r.K = (int)k;
+  r.nr = (int)nr;
+  r.n_ks = n_ks;
+  r.a = reinterpret_cast<const bf16*>(a);
+  r.a_sk = a_sk;
+  r.a_sj = a_sj;
+  r.part = reinterpret_cast<float*>(part);
+  r.nblk = nblk;
+  r.rank = (int)rank;
+  r.alpha = alpha;
+  r.y = reinterpret_cast<bf16*>(y);
+  r.ldy = ldy;
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 sgrid((unsigned)((m + kLdRows - 1) / kLdRows), (unsigned)n_ks, (unsigned)((nr + 63) / 64));
+  if (kmajor)
+    hipLaunchKernelGGL(lora_shrink_kernel<true>, sgrid, dim3(512), 0, st, r);
+  else
+    hipLaunchKernelGGL(lora_shrink_kernel<false>, sgrid, dim3(512), 0, st, r);
+  SWL_LAUNCH_CHECK("lora_shrink_kernel launch");
+  // rows of an expand workgroup: 64, fewer where that leaves CUs idle (each
+  // workgroup reads its columns' B again)
+  const int64_t cgroups = (r.tile0[nblk] + 3) / 4;
+  const int rt = m <= 16 || cgroups * ((m + 31) / 32) < cu_count() ? 1 : cgroups * ((m + 63) / 64) < cu_count() ? 2 : 4;
+  const dim3 egrid((unsigned)cgroups, (unsigned)((m + 16 * rt - 1) / (16 * rt)));
+  const int ksn = rank <= 32 ? 1 : 2;
+  const size_t lds = (size_t)16 * rt * (nr + 8) * 2 + (size_t)4 * 8 * ksn * kLdQuad;
+  switch (ksn * 8 + rt) {
+    case 9: hipLaunchKernelGGL((lora_expand_mfma_kernel<1, 1>), egrid, dim3(256), lds, st, r); break;
+    case 10: hipLaunchKernelGGL((lora_expand_mfma_kernel<1, 2>), egrid, dim3(256), lds, st, r); break;
+    case 12: hipLaunchKernelGGL((lora_expand_mfma_kernel<1, 4>), egrid, dim3(256), lds, st, r); break;
+    case 17: hipLaunchKernelGGL((lora_expand_mfma_kernel<2, 1>), egrid, dim3(256), lds, st, r); break;
+    case 18: hipLaunchKernelGGL((lora_expand_mfma_kernel<2, 2>), egrid, dim3(256), lds, st, r); break;
+    default: hipLaunchKernelGGL((lora_expand_mfma_kernel<2, 4>), egrid, dim3(256), lds, st, r); break;
+  }
+  SWL_LAUNCH_CHECK("lora_expand_mfma_kernel launch");
   return SWL_OK;
 }
 

@@ -413,14 +413,9 @@ LORA_ROWS_MAX = 4      # token rows of one lora_rows launch
 LORA_ROWS_MAX_NR = 64  # shrink columns (blocks x rank)
 
 
-def lora_rows(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int, alpha: float = 1.0,
-              out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """A worker's LoRA delta in one launch (swl_lora_rows_bf16):
-    u = bf16(x @ A) with A = a ([k, nr], a_kmajor) or a.T (a is [nr, k]),
-    then per column block (b, cols, rr_major): bf16(alpha * u[:, blk*rank:
-    (blk+1)*rank] @ B) where B is b [rank, cols] (rr_major, e.g. a diagonal
-    block of fused_B) or b.T (b is [cols, rank], e.g. lora_B).  x is [m, k]
-    with m <= LORA_ROWS_MAX; returns [m, sum(cols)]."""
+def _lora_args(x, a, a_kmajor, blocks):
+    """Shared arguments of lora_rows and lora_delta: (m, k, nr, total columns,
+    A's strides, the blocks' arrays)."""
     _need(x, "x")
     _need(a, "a")
     if x.dim() != 2 or x.stride(1) != 1:
@@ -434,21 +429,68 @@ def lora_rows(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, ra
     srr = (ctypes.c_int64 * n)()
     sc = (ctypes.c_int64 * n)()
     cols = (ctypes.c_int64 * n)()
+    total = 0
     for i, (b, c, rr_major) in enumerate(blocks):
         _need(b, "b")
         ptrs[i] = b.data_ptr()
-        if rr_major:
-            srr[i], sc[i] = b.stride(0), b.stride(1)
-        else:
-            srr[i], sc[i] = b.stride(1), b.stride(0)
+        srr[i], sc[i] = b.stride() if rr_major else b.stride()[::-1]
         cols[i] = int(c)
-    total = int(sum(int(c) for _, c, _ in blocks))
+        total += int(c)
+    ask, asj = a.stride() if a_kmajor else a.stride()[::-1]
+    return m, k, nr, total, ask, asj, (n, ptrs, srr, sc, cols)
+
+
+def lora_rows(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int, alpha: float = 1.0,
+              out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A worker's LoRA delta in one launch (swl_lora_rows_bf16):
+    u = bf16(x @ A) with A = a ([k, nr], a_kmajor) or a.T (a is [nr, k]),
+    then per column block (b, cols, rr_major): bf16(alpha * u[:, blk*rank:
+    (blk+1)*rank] @ B) where B is b [rank, cols] (rr_major, e.g. a diagonal
+    block of fused_B) or b.T (b is [cols, rank], e.g. lora_B).  x is [m, k]
+    with m <= LORA_ROWS_MAX; returns [m, sum(cols)]."""
+    m, k, nr, total, ask, asj, (n, ptrs, srr, sc, cols) = _lora_args(x, a, a_kmajor, blocks)
     if out is None:
         out = torch.empty(m, total, dtype=BF16, device=x.device)
     _lib.check(_lib.load().swl_lora_rows_bf16(
-        _ptr(x), x.stride(0), m, k, _ptr(a), a.stride(0) if a_kmajor else a.stride(1),
-        a.stride(1) if a_kmajor else a.stride(0), nr, n, int(rank), ptrs, srr, sc, cols, float(alpha), _ptr(out),
-        out.stride(0), _stream()))
+        x.data_ptr(), x.stride(0), m, k, a.data_ptr(), ask, asj, nr, n, int(rank), ptrs, srr, sc, cols, float(alpha),
+        out.data_ptr(), out.stride(0), _stream()))
+    return out
+
+
+def lora_delta_fits(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int) -> bool:
+    """Whether lora_delta takes these operands: ranks that are multiples of 8
+    up to 64 (whole 16-byte pieces, one or two MFMA steps), every operand in
+    16-byte aligned rows."""
+    n = len(blocks)
+    nr, ka = (a.shape[1], a.shape[0]) if a_kmajor else a.shape
+    if not (0 < n <= 4 and rank % 8 == 0 and 8 <= rank <= 64 and nr == n * rank and 0 < x.shape[0] <= 1 << 20):
+        return False
+    k = x.shape[1]
+    if k % 8 or k != ka or k > 1 << 20 or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or a.stride(1) != 1 or \
+            a.stride(0) % 8 or a.stride(0) < a.shape[1] or (x.data_ptr() | a.data_ptr()) % 16:
+        return False
+    for b, c, rr_major in blocks:
+        if b.stride(1) != 1 or b.stride(0) % 8 or b.stride(0) < b.shape[1] or b.data_ptr() % 16 or c > 1 << 24 or \
+                (rr_major and c % 8):
+            return False
+    return True
+
+
+def lora_delta(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int, alpha: float = 1.0,
+               out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """lora_rows for any number of rows, in two launches
+    (swl_lora_delta_bf16); lora_delta_fits says which operands it takes."""
+    m, k, nr, total, ask, asj, (n, ptrs, srr, sc, cols) = _lora_args(x, a, a_kmajor, blocks)
+    if out is None:
+        out = torch.empty(m, total, dtype=BF16, device=x.device)
+    # K-slices of the shrink: about 96 workgroups of 32 rows x 64 columns of
+    # A, each with at least 16 k-steps of 32 for its 8 waves
+    groups = -(-m // 32) * -(-nr // 64)
+    n_ks = max(1, min(16, 96 // groups, k // 512))
+    part = torch.empty(n_ks * m * nr, dtype=torch.float32, device=x.device)
+    _lib.check(_lib.load().swl_lora_delta_bf16(
+        x.data_ptr(), x.stride(0), m, k, a.data_ptr(), ask, asj, nr, n, int(rank), ptrs, srr, sc, cols, float(alpha),
+        out.data_ptr(), out.stride(0), part.data_ptr(), n_ks, _stream()))
     return out
 
 

@@ -99,8 +99,11 @@ class SyncRemoteLoRALinear(nn.Module):
         token's few rows take one lora_rows launch."""
         x2 = _as2d(self.dropout(x))
         A, B = self.lora_A.weight.data, self.lora_B.weight.data
+        blocks = [(B, B.shape[0], False)]
         if _rows_fit(x2, A.shape[0]):
-            y = ops.lora_rows(x2, A, False, [(B, B.shape[0], False)], A.shape[0], float(self.scaling))
+            y = ops.lora_rows(x2, A, False, blocks, A.shape[0], float(self.scaling))
+        elif ops.lora_delta_fits(x2, A, False, blocks, A.shape[0]):
+            y = ops.lora_delta(x2, A, False, blocks, A.shape[0], float(self.scaling))
         else:
             u = self.lora_A(x2)
             y = ops.matmul(u, B, trans_b=True, alpha=float(self.scaling))
@@ -150,20 +153,22 @@ class FusedLoRA(nn.Module):
             return [None] * self.num_loras
         x2 = _as2d(self.dropout(x))
         fA, fB, r = self.fused_A.data, self.fused_B.data, self.rank
-        if _rows_fit(x2, fA.shape[1]) and len(self.out_dims) <= 4:
+        blocks, col = [], 0
+        for i, d in enumerate(self.out_dims):
+            blocks.append((fB[i * r:(i + 1) * r, col:col + d], d, True))
+            col += d
+        if _rows_fit(x2, fA.shape[1]) and len(blocks) <= 4:
             # a decode token's rows: shrink and every block's expand in one launch
-            blocks, col = [], 0
-            for i, d in enumerate(self.out_dims):
-                blocks.append((fB[i * r:(i + 1) * r, col:col + d], d, True))
-                col += d
             delta = ops.lora_rows(x2, fA, True, blocks, r)
+        elif ops.lora_delta_fits(x2, fA, True, blocks, r):
+            # a prompt chunk: one launch each
+            delta = ops.lora_delta(x2, fA, True, blocks, r)
         else:
             u = ops.matmul(x2, fA, trans_b=False)            # [m, n*r] bf16
             delta = torch.empty(x2.shape[0], sum(self.out_dims), dtype=x2.dtype, device=x2.device)
             col = 0
-            for i, d in enumerate(self.out_dims):
-                ops.matmul(u[:, i * r:(i + 1) * r], fB[i * r:(i + 1) * r, col:col + d], trans_b=False,
-                           out=delta[:, col:col + d])
+            for i, (b, d, _) in enumerate(blocks):
+                ops.matmul(u[:, i * r:(i + 1) * r], b, trans_b=False, out=delta[:, col:col + d])
                 col += d
         delta = delta.reshape(*x.shape[:-1], delta.shape[-1])
         return list(delta.split(self.out_dims, dim=-1))
