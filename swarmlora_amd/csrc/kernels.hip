@@ -2094,6 +2094,186 @@ __global__ __launch_bounds__(256) void lora_rows_kernel(LoraRowsArgs a) {
   }
 }
 
+// The same for ranks 8, 16, 32 and 64 in 16-byte aligned rows: 1024 threads a
+// workgroup, which computes the shrink of its own column block only (rank
+// columns of A, not nr) and then 1024 output columns of it.  The kernel above
+// is bound by each workgroup's chain of A loads (256 threads over all of A:
+// 24-51 us a delta at K = 4096 and 14336, rank 16, one row); here A is one or
+// a few batches of 8 loads a thread, and its share of B is requested before
+// the shrink: 6-10 us.  Still one launch: on a GPU that many worker processes
+// share, a dependent launch costs more than the repeated reads of A, which
+// come from L2.
+constexpr int kLrCols = 1024;  // output columns of a workgroup
+struct LoraWideArgs {
+  LoraRowsArgs r;
+  int wg0[kLoraRowsMaxBlk + 1];  // first workgroup of block b
+  int kc;                        // K elements staged at a time
+};
+template <bool KMAJOR, int M>  // A as [k][j] rows; rows of x (at most)
+__global__ __launch_bounds__(1024) void lora_rows_wide_kernel(LoraWideArgs w) {
+  const LoraRowsArgs& a = w.r;
+  extern __shared__ __attribute__((aligned(16))) char lr_lds[];
+  __shared__ float red[16][M][64];
+  __shared__ float us[M][64];
+  bf16* xs = reinterpret_cast<bf16*>(lr_lds);  // [M][kc], then B's partial sums [8][kLrCols]
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int b = 0;
+  while (b + 1 < a.nblk && (int)blockIdx.x >= w.wg0[b + 1]) ++b;
+  const int64_t c0 = (int64_t)((int)blockIdx.x - w.wg0[b]) * kLrCols;  // in the block
+  const int nc = (int)min<int64_t>(kLrCols, a.off[b + 1] - a.off[b] - c0);
+  const int ro = a.rank >> 3;  // 1, 2, 4 or 8
+  const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+
+  // this thread's share of B: rows of columns: rr = rg * ro .. + ro - 1 of 8
+  // columns; columns of ranks: column tid
+  const bool brows = a.sc[b] == 1;
+  const int rg = tid >> 7, oc = 8 * (tid & 127);
+  u32x4 bv[8];
+  auto load_b = [&]() {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (i >= ro) break;
+      bv[i] = brows ? (oc < nc ? ldg16(a.b[b] + (rg * ro + i) * a.srr[b] + c0 + oc) : zero)
+                    : (tid < nc ? ldg16(a.b[b] + (c0 + tid) * a.sc[b] + 8 * i) : zero);
+    }
+  };
+  if constexpr (M == 1) load_b();  // (with more rows the registers do not hold it)
+
+  const bf16* A = a.a + (int64_t)b * a.rank * a.a_sj;
+  // KMAJOR: thread (octet o of the block's columns, k-partition p)
+  const int lg = __builtin_ctz(ro), o = tid & (ro - 1), p = tid >> lg, P = 1024 >> lg;
+  // else: wave -> columns j = wv, wv + 16, .. (rank 8: column wv % 8, half wv / 8 of K)
+  const int kp = a.rank >= 16 ? 1 : 2, j0 = kp == 1 ? wv : wv & 7, part = kp == 1 ? 0 : wv >> 3;
+  const int ncol = a.rank >= 16 ? a.rank >> 4 : 1;
+  constexpr int U = M == 1 ? 8 : 4;  // loads of A in flight
+  float acc[M][8];                   // KMAJOR: the octet
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[m][i] = 0.f;
+  if constexpr (!KMAJOR)
+    for (int i = tid; i < 2 * M * 64; i += 1024) (&red[0][0][0])[i] = 0.f;
+
+  for (int64_t k0 = 0; k0 < a.K; k0 += w.kc) {
+    const int kc = (int)min<int64_t>(w.kc, a.K - k0), k8 = kc >> 3;
+    if (k0 > 0) __syncthreads();
+    for (int m = 0; m < a.m; ++m)
+      for (int i = tid; i < k8; i += 1024)
+        *reinterpret_cast<u32x4*>(xs + m * w.kc + 8 * i) = ldg16(a.x + m * a.ldx + k0 + 8 * i);
+    if constexpr (KMAJOR) {
+      const bf16* Ak = A + k0 * a.a_sk + 8 * o;
+      for (int kb = p; kb < kc + p; kb += U * P) {  // as often in every thread
+        u32x4 av[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) av[u] = kb + u * P < kc ? ldg16(Ak + (int64_t)(kb + u * P) * a.a_sk) : zero;
+        if (kb == p) __syncthreads();  // x is staged
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (kb + u * P >= kc) break;
+          float av8[8];
+          unpack8(av[u], av8);
+#pragma unroll
+          for (int m = 0; m < M; ++m) {
+            const float xv = bf2f(xs[m * w.kc + kb + u * P]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[m][i] += xv * av8[i];
+          }
+        }
+      }
+    } else {
+      const int i0 = part * 64 + lane;
+#pragma unroll 1
+      for (int c = 0; c < ncol; ++c) {
+        const bf16* Ak = A + (int64_t)(j0 + 16 * c) * a.a_sj + k0;
+        float v[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) v[m] = 0.f;
+#pragma unroll 1
+        for (int ib = i0; ib < k8 + i0; ib += U * 64 * kp) {
+          u32x4 av[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) av[u] = ib + u * 64 * kp < k8 ? ldg16(Ak + 8 * (ib + u * 64 * kp)) : zero;
+          if (c == 0 && ib == i0) __syncthreads();  // x is staged
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            if (ib + u * 64 * kp >= k8) break;
+            float av8[8];
+            unpack8(av[u], av8);
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+              float xv[8];
+              unpack8(lds16(xs + m * w.kc + 8 * (ib + u * 64 * kp)), xv);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) v[m] += xv[i] * av8[i];
+            }
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+#pragma unroll
+          for (int d = 32; d >= 1; d >>= 1) v[m] += __shfl_xor(v[m], d, 64);
+          if (lane == 0) red[part][m][j0 + 16 * c] += v[m];  // (this wave's own entry)
+        }
+      }
+    }
+  }
+  if constexpr (M > 1) load_b();
+  if constexpr (KMAJOR) {  // over the lanes of the same octet
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      for (int d = ro; d < 64; d <<= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[m][i] += __shfl_xor(acc[m][i], d, 64);
+      if (lane < ro)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) red[wv][m][8 * lane + i] = acc[m][i];
+    }
+  }
+  __syncthreads();
+  if (tid < M * a.rank) {
+    const int m = tid / a.rank, j = tid - m * a.rank;
+    float v = red[0][m][j];
+    for (int q = 1; q < (KMAJOR ? 16 : kp); ++q) v += red[q][m][j];
+    us[m][j] = bf2f(f2bf(v));
+  }
+  __syncthreads();
+  float* ps = reinterpret_cast<float*>(lr_lds);
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    if (m >= a.m) break;
+    float v = 0.f;
+    if (brows) {
+      float v8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i >= ro) break;
+        float bf[8];
+        unpack8(bv[i], bf);
+        const float u = us[m][rg * ro + i];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v8[e] += u * bf[e];
+      }
+      if (m > 0) __syncthreads();
+#pragma unroll
+      for (int e = 0; e < 8; e += 4)
+        *reinterpret_cast<f32x4*>(ps + rg * kLrCols + oc + e) = f32x4{v8[e], v8[e + 1], v8[e + 2], v8[e + 3]};
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v += ps[q * kLrCols + tid];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i >= ro) break;
+        float bf[8];
+        unpack8(bv[i], bf);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v += us[m][8 * i + e] * bf[e];
+      }
+    }
+    if (tid < nc) stg(a.y + m * a.ldy + a.off[b] + c0 + tid, f2bf(a.alpha * v));
+  }
+}
+
 // LoRA delta of a worker's prompt chunk (more rows than lora_rows takes) in
 // two launches: lora_shrink_kernel, then lora_expand_mfma_kernel.  As scalar
 // products, one output a thread, a layer's four deltas of 512 rows took 999
@@ -5123,8 +5303,36 @@ int swl_lora_rows_bf16(const void* x, int64_t ldx, int64_t m, int64_t k, const v
   r.alpha = alpha;
   r.y = reinterpret_cast<bf16*>(y);
   r.ldy = ldy;
-  const unsigned grid = (unsigned)std::min<int64_t>(32, std::max<int64_t>(1, (r.off[nblk] + 1023) / 1024));
   hipStream_t st = (hipStream_t)stream;
+  // the wide kernel: ranks of whole octets that divide its threads, A and
+  // every B in 16-byte aligned rows
+  bool wide = (rank == 8 || rank == 16 || rank == 32 || rank == 64) && r.a_mode <= 1;
+  LoraWideArgs w{};
+  for (int i = 0; i < nblk; ++i) {
+    const bool rows = b_sc[i] == 1;
+    wide = wide && (reinterpret_cast<uintptr_t>(b[i]) & 15) == 0 &&
+           (rows ? b_srr[i] % 8 == 0 && blk_cols[i] % 8 == 0 : b_srr[i] == 1 && b_sc[i] % 8 == 0) &&
+           r.off[nblk] < ((int64_t)1 << 31);
+    w.wg0[i + 1] = w.wg0[i] + (int)((blk_cols[i] + kLrCols - 1) / kLrCols);
+  }
+  if (wide) {
+    w.r = r;
+    const int rows = m == 1 ? 1 : kLoraRowsMaxRows;
+    w.kc = (int)std::min<int64_t>(k, 32 * 1024 / 2 / rows);  // 32 KiB of x
+    const size_t lds = std::max<size_t>((size_t)rows * w.kc * 2, 8 * kLrCols * sizeof(float));
+    const dim3 wgrid((unsigned)w.wg0[nblk]);
+    if (m == 1 && r.a_mode == 1)
+      hipLaunchKernelGGL((lora_rows_wide_kernel<true, 1>), wgrid, dim3(1024), lds, st, w);
+    else if (m == 1)
+      hipLaunchKernelGGL((lora_rows_wide_kernel<false, 1>), wgrid, dim3(1024), lds, st, w);
+    else if (r.a_mode == 1)
+      hipLaunchKernelGGL((lora_rows_wide_kernel<true, kLoraRowsMaxRows>), wgrid, dim3(1024), lds, st, w);
+    else
+      hipLaunchKernelGGL((lora_rows_wide_kernel<false, kLoraRowsMaxRows>), wgrid, dim3(1024), lds, st, w);
+    SWL_LAUNCH_CHECK("lora_rows_wide_kernel launch");
+    return SWL_OK;
+  }
+  const unsigned grid = (unsigned)std::min<int64_t>(32, std::max<int64_t>(1, (r.off[nblk] + 1023) / 1024));
   if (nr <= 16)
     hipLaunchKernelGGL(lora_rows_kernel<16>, dim3(grid), dim3(256), 0, st, r);
   else if (nr <= 32)

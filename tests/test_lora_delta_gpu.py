@@ -91,3 +91,27 @@ def test_worker_modules_route_by_rank(dev, t, rank):
     for g, (a, b) in zip(got, ab):
         assert_close(g[0], _want(x[0], (a * 2).t(), [b.t()], rank, 1.0), what="fused")
     assert_close(one[0], _want(x[0], ab[0][0].t(), [ab[0][1].t()], rank, 2.0), what="remote")
+
+
+@pytest.mark.parametrize("m,k,rank,cols,kmajor,rr_major", [
+    (1, 4096, 16, [4096, 1024, 1024], True, True), (1, 4096, 16, [14336, 14336], True, True),
+    (1, 14336, 16, [4096], False, False), (1, 4096, 64, [1000], False, False), (1, 8, 8, [8], True, True),
+    (1, 24, 8, [1025], False, False), (1, 16384, 8, [1032, 24], True, True), (1, 16392, 32, [2056, 16], True, True),
+    (1, 20000, 64, [1024], False, False), (2, 4096, 8, [1024, 8, 2048], True, True), (3, 4104, 32, [520, 520], True, True),
+    (4, 14336, 64, [1023], False, False), (4, 8200, 16, [64, 1024, 16, 8], True, True), (4, 4096, 64, [136], True, False),
+    (2, 1000, 16, [264], False, True),
+])
+def test_lora_rows_wide_matches_two_products(dev, m, k, rank, cols, kmajor, rr_major):
+    """The one-launch delta of a few rows in the ranks and layouts of its
+    wide kernel: 1024-column workgroups, K staged in pieces, every rank."""
+    from swarmlora_amd import ops
+    n = len(cols)
+    x, fA = randn((m, k), 1), randn((k, n * rank), 2, std=0.05)
+    bs = [randn((rank, c), 3 + i, std=0.05) for i, c in enumerate(cols)]
+    a = fA.to(dev) if kmajor else fA.t().contiguous().to(dev)
+    blocks = [(b.to(dev) if rr_major else b.t().contiguous().to(dev), c, rr_major) for b, c in zip(bs, cols)]
+    buf = torch.full((m + 1, sum(cols) + 24), 7.0, dtype=BF16, device=dev)
+    ops.lora_rows(x.to(dev), a, kmajor, blocks, rank, 2.0, out=buf[:m, :sum(cols)])
+    torch.cuda.synchronize()
+    assert_close(buf[:m, :sum(cols)], _want(x, fA, bs, rank, 2.0), what="lora_rows")
+    assert bool((buf[m:] == 7.0).all()) and bool((buf[:, sum(cols):] == 7.0).all())
