@@ -413,84 +413,133 @@ LORA_ROWS_MAX = 4      # token rows of one lora_rows launch
 LORA_ROWS_MAX_NR = 64  # shrink columns (blocks x rank)
 
 
-def _lora_args(x, a, a_kmajor, blocks):
-    """Shared arguments of lora_rows and lora_delta: (m, k, nr, total columns,
-    A's strides, the blocks' arrays)."""
+class LoraBlocks:
+    """The column blocks of one LoRA delta as lora_rows and lora_delta take
+    them, built per call from plain numbers: addresses, rank strides, column
+    strides and columns of each block's B, in one host array."""
+
+    __slots__ = ("n", "vals", "total")
+
+    def __init__(self, ptrs: list, srr: list, sc: list, cols: list):
+        self.n = len(ptrs)
+        self.vals = ptrs + srr + sc + cols
+        self.total = sum(cols)
+
+    @classmethod
+    def of(cls, blocks: list) -> "LoraBlocks":
+        """blocks: (b, cols, rr_major) each, B = b [rank, cols] (rr_major) or
+        b.T (b is [cols, rank])."""
+        ptrs, srr, sc, cols = [], [], [], []
+        for b, c, rr_major in blocks:
+            _need(b, "b")
+            s0, s1 = b.stride()
+            ptrs.append(b.data_ptr())
+            srr.append(s0 if rr_major else s1)
+            sc.append(s1 if rr_major else s0)
+            cols.append(int(c))
+        return cls(ptrs, srr, sc, cols)
+
+    @classmethod
+    def diagonal(cls, b: torch.Tensor, rank: int, dims: list) -> "LoraBlocks":
+        """The diagonal blocks of a fused B [len(dims) * rank, sum(dims)]:
+        block i is its rows i * rank .. and the columns of dims[i]."""
+        _need(b, "b")
+        n = len(dims)
+        if b.dim() != 2 or b.shape[0] < n * rank or b.shape[1] < sum(dims):
+            raise ValueError("fused B must be [blocks * rank, sum of the blocks' columns]")
+        p, (s0, s1) = b.data_ptr(), b.stride()
+        ptrs, col = [], 0
+        for i, d in enumerate(dims):
+            ptrs.append(p + 2 * (i * rank * s0 + col * s1))
+            col += d
+        return cls(ptrs, [s0] * n, [s1] * n, list(dims))
+
+    def vectors(self, rank: int) -> bool:
+        """Every B in 16-byte aligned rows, of whole 16-byte pieces where the
+        rows are columns."""
+        n, v = self.n, self.vals
+        for i in range(n):
+            p, srr, sc, c = v[i], v[n + i], v[2 * n + i], v[3 * n + i]
+            if p % 16 or c > 1 << 24 or not (srr % 8 == 0 and srr >= c and c % 8 == 0 if sc == 1 else
+                                             srr == 1 and sc % 8 == 0 and sc >= rank):
+                return False
+        return True
+
+
+def _lora_call(x, a, a_kmajor, blocks):
+    """Checks and leading arguments of lora_rows / lora_delta: (blocks, m, k,
+    nr, A's stride over k, over columns)."""
     _need(x, "x")
     _need(a, "a")
+    if not isinstance(blocks, LoraBlocks):
+        blocks = LoraBlocks.of(blocks)
     if x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("lora_rows: x must be 2-D with unit column stride")
     m, k = x.shape
-    nr = a.shape[1] if a_kmajor else a.shape[0]
-    if (a.shape[0] if a_kmajor else a.shape[1]) != k:
+    a0, a1 = a.shape
+    s0, s1 = a.stride()
+    if not a_kmajor:
+        a0, a1, s0, s1 = a1, a0, s1, s0
+    if a0 != k:
         raise ValueError("lora_rows: A does not match x")
-    n = len(blocks)
-    ptrs = (ctypes.c_void_p * n)()
-    srr = (ctypes.c_int64 * n)()
-    sc = (ctypes.c_int64 * n)()
-    cols = (ctypes.c_int64 * n)()
-    total = 0
-    for i, (b, c, rr_major) in enumerate(blocks):
-        _need(b, "b")
-        ptrs[i] = b.data_ptr()
-        srr[i], sc[i] = b.stride() if rr_major else b.stride()[::-1]
-        cols[i] = int(c)
-        total += int(c)
-    ask, asj = a.stride() if a_kmajor else a.stride()[::-1]
-    return m, k, nr, total, ask, asj, (n, ptrs, srr, sc, cols)
+    return blocks, m, k, a1, s0, s1
 
 
-def lora_rows(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int, alpha: float = 1.0,
+def lora_rows(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks, rank: int, alpha: float = 1.0,
               out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """A worker's LoRA delta in one launch (swl_lora_rows_bf16):
     u = bf16(x @ A) with A = a ([k, nr], a_kmajor) or a.T (a is [nr, k]),
     then per column block (b, cols, rr_major): bf16(alpha * u[:, blk*rank:
     (blk+1)*rank] @ B) where B is b [rank, cols] (rr_major, e.g. a diagonal
-    block of fused_B) or b.T (b is [cols, rank], e.g. lora_B).  x is [m, k]
-    with m <= LORA_ROWS_MAX; returns [m, sum(cols)]."""
-    m, k, nr, total, ask, asj, (n, ptrs, srr, sc, cols) = _lora_args(x, a, a_kmajor, blocks)
+    block of fused_B) or b.T (b is [cols, rank], e.g. lora_B); blocks: a list
+    of those or a LoraBlocks.  x is [m, k] with m <= LORA_ROWS_MAX; returns
+    [m, sum(cols)]."""
+    blocks, m, k, nr, ask, asj = _lora_call(x, a, a_kmajor, blocks)
+    n = blocks.n
     if out is None:
-        out = torch.empty(m, total, dtype=BF16, device=x.device)
+        out = torch.empty((m, blocks.total), dtype=BF16, device=x.device)
+    v = (ctypes.c_int64 * (4 * n))(*blocks.vals)
+    p = ctypes.addressof(v)
     _lib.check(_lib.load().swl_lora_rows_bf16(
-        x.data_ptr(), x.stride(0), m, k, a.data_ptr(), ask, asj, nr, n, int(rank), ptrs, srr, sc, cols, float(alpha),
-        out.data_ptr(), out.stride(0), _stream()))
+        x.data_ptr(), x.stride(0), m, k, a.data_ptr(), ask, asj, nr, n, int(rank), p, p + 8 * n, p + 16 * n,
+        p + 24 * n, float(alpha), out.data_ptr(), out.stride(0), _stream()))
     return out
 
 
-def lora_delta_fits(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int) -> bool:
+def lora_delta_fits(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks, rank: int) -> bool:
     """Whether lora_delta takes these operands: ranks that are multiples of 8
     up to 64 (whole 16-byte pieces, one or two MFMA steps), every operand in
     16-byte aligned rows."""
-    n = len(blocks)
+    if not isinstance(blocks, LoraBlocks):
+        blocks = LoraBlocks.of(blocks)
+    n = blocks.n
     nr, ka = (a.shape[1], a.shape[0]) if a_kmajor else a.shape
     if not (0 < n <= 4 and rank % 8 == 0 and 8 <= rank <= 64 and nr == n * rank and 0 < x.shape[0] <= 1 << 20):
         return False
-    k = x.shape[1]
-    if k % 8 or k != ka or k > 1 << 20 or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or a.stride(1) != 1 or \
-            a.stride(0) % 8 or a.stride(0) < a.shape[1] or (x.data_ptr() | a.data_ptr()) % 16:
+    k, (x0, x1), (a0, a1) = x.shape[1], x.stride(), a.stride()
+    if k % 8 or k != ka or k > 1 << 20 or x1 != 1 or x0 % 8 or x0 < k or a1 != 1 or a0 % 8 or a0 < a.shape[1] or \
+            (x.data_ptr() | a.data_ptr()) % 16:
         return False
-    for b, c, rr_major in blocks:
-        if b.stride(1) != 1 or b.stride(0) % 8 or b.stride(0) < b.shape[1] or b.data_ptr() % 16 or c > 1 << 24 or \
-                (rr_major and c % 8):
-            return False
-    return True
+    return blocks.vectors(rank)
 
 
-def lora_delta(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks: list, rank: int, alpha: float = 1.0,
+def lora_delta(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks, rank: int, alpha: float = 1.0,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """lora_rows for any number of rows, in two launches
     (swl_lora_delta_bf16); lora_delta_fits says which operands it takes."""
-    m, k, nr, total, ask, asj, (n, ptrs, srr, sc, cols) = _lora_args(x, a, a_kmajor, blocks)
+    blocks, m, k, nr, ask, asj = _lora_call(x, a, a_kmajor, blocks)
+    n = blocks.n
     if out is None:
-        out = torch.empty(m, total, dtype=BF16, device=x.device)
+        out = torch.empty((m, blocks.total), dtype=BF16, device=x.device)
     # K-slices of the shrink: about 96 workgroups of 32 rows x 64 columns of
     # A, each with at least 16 k-steps of 32 for its 8 waves
-    groups = -(-m // 32) * -(-nr // 64)
-    n_ks = max(1, min(16, 96 // groups, k // 512))
+    n_ks = max(1, min(16, 96 // max(1, -(-m // 32) * -(-nr // 64)), k // 512))
     part = torch.empty(n_ks * m * nr, dtype=torch.float32, device=x.device)
+    v = (ctypes.c_int64 * (4 * n))(*blocks.vals)
+    p = ctypes.addressof(v)
     _lib.check(_lib.load().swl_lora_delta_bf16(
-        x.data_ptr(), x.stride(0), m, k, a.data_ptr(), ask, asj, nr, n, int(rank), ptrs, srr, sc, cols, float(alpha),
-        out.data_ptr(), out.stride(0), part.data_ptr(), n_ks, _stream()))
+        x.data_ptr(), x.stride(0), m, k, a.data_ptr(), ask, asj, nr, n, int(rank), p, p + 8 * n, p + 16 * n,
+        p + 24 * n, float(alpha), out.data_ptr(), out.stride(0), part.data_ptr(), n_ks, _stream()))
     return out
 
 

@@ -99,11 +99,11 @@ class SyncRemoteLoRALinear(nn.Module):
         token's few rows take one lora_rows launch."""
         x2 = _as2d(self.dropout(x))
         A, B = self.lora_A.weight.data, self.lora_B.weight.data
-        blocks = [(B, B.shape[0], False)]
-        if _rows_fit(x2, A.shape[0]):
-            y = ops.lora_rows(x2, A, False, blocks, A.shape[0], float(self.scaling))
-        elif ops.lora_delta_fits(x2, A, False, blocks, A.shape[0]):
-            y = ops.lora_delta(x2, A, False, blocks, A.shape[0], float(self.scaling))
+        blocks, r = ops.LoraBlocks.of([(B, B.shape[0], False)]), A.shape[0]
+        if _rows_fit(x2, r):
+            y = ops.lora_rows(x2, A, False, blocks, r, float(self.scaling))
+        elif ops.lora_delta_fits(x2, A, False, blocks, r):
+            y = ops.lora_delta(x2, A, False, blocks, r, float(self.scaling))
         else:
             u = self.lora_A(x2)
             y = ops.matmul(u, B, trans_b=True, alpha=float(self.scaling))
@@ -153,11 +153,8 @@ class FusedLoRA(nn.Module):
             return [None] * self.num_loras
         x2 = _as2d(self.dropout(x))
         fA, fB, r = self.fused_A.data, self.fused_B.data, self.rank
-        blocks, col = [], 0
-        for i, d in enumerate(self.out_dims):
-            blocks.append((fB[i * r:(i + 1) * r, col:col + d], d, True))
-            col += d
-        if _rows_fit(x2, fA.shape[1]) and len(blocks) <= 4:
+        blocks = ops.LoraBlocks.diagonal(fB, r, self.out_dims)
+        if _rows_fit(x2, fA.shape[1]) and blocks.n <= 4:
             # a decode token's rows: shrink and every block's expand in one launch
             delta = ops.lora_rows(x2, fA, True, blocks, r)
         elif ops.lora_delta_fits(x2, fA, True, blocks, r):
@@ -167,8 +164,9 @@ class FusedLoRA(nn.Module):
             u = ops.matmul(x2, fA, trans_b=False)            # [m, n*r] bf16
             delta = torch.empty(x2.shape[0], sum(self.out_dims), dtype=x2.dtype, device=x2.device)
             col = 0
-            for i, (b, d, _) in enumerate(blocks):
-                ops.matmul(u[:, i * r:(i + 1) * r], b, trans_b=False, out=delta[:, col:col + d])
+            for i, d in enumerate(self.out_dims):
+                ops.matmul(u[:, i * r:(i + 1) * r], fB[i * r:(i + 1) * r, col:col + d], trans_b=False,
+                           out=delta[:, col:col + d])
                 col += d
         delta = delta.reshape(*x.shape[:-1], delta.shape[-1])
         return list(delta.split(self.out_dims, dim=-1))
