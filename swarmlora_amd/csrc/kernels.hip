@@ -1319,6 +1319,13 @@ struct TiledArgs {
   // gemm256_kernel: LoRA delta as MFMA k-steps (every tile inside one column
   // block, ranks multiples of 8 up to 64) instead of in the epilogue
   int32_t lora_mfma;
+  // K split over n_split workgroups per tile (1: none), their fp32 tiles to
+  // part [n_split][M][N], summed by prefill_fold_kernel
+  int32_t n_split;
+  float* part;
+  // first row of the 128 x 128 tiles: the rows before it have large tiles in
+  // a launch of their own (whose M ends there)
+  int64_t m_base;
 };
 
 // LDS rows of 64 bf16 (eight 16-byte chunks) with the chunks of row r
@@ -1465,18 +1472,20 @@ __global__ __launch_bounds__(256) void tiled_kernel(TiledArgs a) {
 // XCD (workgroup i runs on XCD i % 8) walks a contiguous run of tiles,
 // tokens fastest: the W rows of a tile column are read by the XCD's
 // workgroups together, from its L2.
-constexpr int PG_M = 256, PG_N = 256, PG_K = 64, PG_SLOTS = 2;
+constexpr int PG_M = 256, PG_N = 256, PG_K = 64;  // the largest tile, k per stage
 constexpr int PG_ROW = PG_K * 2;                           // bytes of an LDS row
 constexpr int PG_ELD = 64 + 4;                            // epilogue staging row (fp32)
-// Waves 2 WM: two along the columns (128 each), WM along the token rows; NJ:
-// 32-row MFMA tiles of tokens per wave, so 32 WM NJ token rows a tile (256
-// or 192; W always 256 columns).  Stage: W 256 rows, then x MT rows.
-template <int NJ, int WM>
+// Waves 2 WM: two along the columns (32 NI each), WM along the token rows; NI
+// and NJ: 32-wide MFMA tiles of columns and of tokens per wave, so 64 NI
+// columns and 32 WM NJ token rows a tile: 256 x 256 or 256 x 192 in two slots,
+// 128 x 128 in four (the same bytes in flight).  Stage: W NT rows, then x MT.
+template <int NI, int NJ, int WM, int SLOTS>
 struct PgGeom {
+  static constexpr int NT = 64 * NI;                        // columns of a tile
   static constexpr int MT = 32 * WM * NJ;                   // token rows of a tile
-  static constexpr int STAGE = (PG_N + MT) * PG_ROW;        // 64 or 56 KiB
+  static constexpr int STAGE = (NT + MT) * PG_ROW;          // 64, 56 or 32 KiB
   static constexpr int EPI = 2 * WM * 32 * NJ * PG_ELD * 4; // epilogue staging, one region a wave
-  static constexpr int AREA = PG_SLOTS * STAGE > EPI ? PG_SLOTS * STAGE : EPI;
+  static constexpr int AREA = SLOTS * STAGE > EPI ? SLOTS * STAGE : EPI;
   // then the tile's row table: output row pointer (8 bytes) and epilogue
   // adapter (4 bytes) of each of its token rows; then the LoRA entries
   // (lora_B block pointer, rank, scale) of the segments the tile overlaps
@@ -1495,21 +1504,23 @@ __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
                                                  0, 0, 0);
 }
 
-template <int NJ, int WM>
+template <int NI, int NJ, int WM, int SLOTS>
 __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int tiles_m, int tiles, int per_xcd,
                                                                int gm) {
-  // PG_SLOTS x [W 256 x 64 | x MT x 64]; then the epilogue's WAVES x [TPW][PG_ELD] fp32
-  using Geo = PgGeom<NJ, WM>;
+  // SLOTS x [W NT x 64 | x MT x 64]; then the epilogue's WAVES x [TPW][PG_ELD] fp32
+  using Geo = PgGeom<NI, NJ, WM, SLOTS>;
   constexpr int WAVES = 2 * WM;
+  constexpr int NT = Geo::NT, CPW = 32 * NI;                    // columns: tile, wave
   constexpr int MT = Geo::MT, TPW = 32 * NJ, XR = MT / WAVES;  // token rows: tile, wave, DMA rows a wave
-  constexpr int WR = PG_N / WAVES;                              // W rows a wave moves per stage
-  constexpr int MF = 4 * NJ, NR = 4 + NJ;                       // MFMAs and fragment reads per k-step
+  constexpr int WR = NT / WAVES;                                // W rows a wave moves per stage
+  constexpr int MF = NI * NJ, NR = NI + NJ;                     // MFMAs and fragment reads per k-step
   constexpr int NREQ = WR / 8 + XR / 8;                         // DMA instructions a wave per stage
-  static_assert(PG_N % (8 * WAVES) == 0 && MT % (8 * WAVES) == 0, "the waves' DMA rows must cover the stage");
+  static_assert(WR % 16 == 0 && XR % 16 == 0 && NR <= MF, "the waves' DMA rows must cover the stage");
+  static_assert((SLOTS & (SLOTS - 1)) == 0 && NREQ * (SLOTS - 1) < 64, "slots are a power of two");
   extern __shared__ __attribute__((aligned(16))) char pg_lds[];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wv >> 1, wn = wv & 1;  // wave: tokens wm * TPW.., columns wn * 128..
+  const int wm = wv >> 1, wn = wv & 1;  // wave: tokens wm * TPW.., columns wn * CPW..
   const int lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (lin >= tiles) return;  // uniform over the workgroup
   // linear tile lin: groups of gm row tiles, each group walking its column
@@ -1517,21 +1528,25 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   const int gsz = gm * (tiles / tiles_m);
   const int grp = lin / gsz, gl = lin - grp * gsz;
   const int gr = min(gm, tiles_m - grp * gm);  // row tiles in this group
-  const int64_t m0 = (int64_t)(grp * gm + gl % gr) * MT;
-  const int64_t n0 = (int64_t)(gl / gr) * PG_N;
-  const int nk = (int)(a.K / PG_K);
+  constexpr bool SPLIT = NI == 2;  // (the large tiles keep a loop that knows nothing of splits: 1 % otherwise)
+  const int64_t m0 = (SPLIT ? a.m_base : 0) + (int64_t)(grp * gm + gl % gr) * MT;
+  const int64_t n0 = (int64_t)(gl / gr) * NT;
+  // this workgroup's stages of K (all of them unless K is split)
+  const int sp = SPLIT ? blockIdx.y : 0;
+  const int kt0 = SPLIT ? (int)(a.K / PG_K) * sp / a.n_split : 0;
+  const int nk = SPLIT ? (int)(a.K / PG_K) * (sp + 1) / a.n_split - kt0 : (int)(a.K / PG_K);
 
-  f32x16 acc[4][NJ];
+  f32x16 acc[NI][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   const int fr = lane & 31, fh = lane >> 5;
-  auto mma = [&](const u32x4 (&fa)[4], const u32x4 (&fb)[NJ]) {
+  auto mma = [&](const u32x4 (&fa)[NI], const u32x4 (&fb)[NJ]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < NJ; ++j) acc[i][j] = mfma32(fa[i], fb[j], acc[i][j]);
   };
@@ -1541,7 +1556,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   // the order written here is the order issued.  Spreading the requests
   // keeps the CU's address queue from blocking the wave (a 1 KiB LDS-DMA
   // request takes the queue about 16 cycles).
-  auto mfma_at = [&](u32x4 (&a0)[4], u32x4 (&b0)[NJ], u32x4 (&a1)[4], u32x4 (&b1)[NJ], int t) {
+  auto mfma_at = [&](u32x4 (&a0)[NI], u32x4 (&b0)[NJ], u32x4 (&a1)[NI], u32x4 (&b1)[NJ], int t) {
     const int i = (t % MF) / NJ, j = t % NJ;
     if (t < MF)
       acc[i][j] = mfma32(a0[i], b0[j], acc[i][j]);
@@ -1584,7 +1599,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   for (int i = 0; i < WR / 8; ++i) {
     const int64_t r = WR * wv + 8 * i + dr;
     const int dc = (lane & 7) ^ dr ^ (i & 1);
-    wsrc[i] = a.w + min(n0 + r, a.N - 1) * a.K + 8 * dc;
+    wsrc[i] = a.w + min(n0 + r, a.N - 1) * a.K + (int64_t)kt0 * PG_K + 8 * dc;
   }
 #pragma unroll
   for (int i = 0; i < XR / 8; ++i) {
@@ -1592,10 +1607,10 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
     const int dc = (lane & 7) ^ dr ^ (i & 1);
     const int64_t mr = min(m0 + r, a.M - 1);
     if (a.x) {
-      xsrc[i] = a.x + mr * a.K + 8 * dc;
+      xsrc[i] = a.x + mr * a.K + (int64_t)kt0 * PG_K + 8 * dc;
     } else {  // the token row in its slot buffer (no packed copy)
       const int sg = find_seg(a.out.off, a.out.n, mr);
-      xsrc[i] = a.xin[sg] + (mr - a.out.off[sg]) * a.K + 8 * dc;
+      xsrc[i] = a.xin[sg] + (mr - a.out.off[sg]) * a.K + (int64_t)kt0 * PG_K + 8 * dc;
     }
   }
   // DMA instruction q of a stage (W 0 .. WR / 8 - 1, then x): into slot s
@@ -1607,7 +1622,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
                                        (lds_ptr)(st + (WR * wv + 8 * q) * PG_ROW), 16, 0, 0);
     else
       __builtin_amdgcn_global_load_lds((gbl_ptr)(xsrc[q - QW] + (int64_t)kt * PG_K),
-                                       (lds_ptr)(st + PG_N * PG_ROW + (XR * wv + 8 * (q - QW)) * PG_ROW), 16, 0, 0);
+                                       (lds_ptr)(st + NT * PG_ROW + (XR * wv + 8 * (q - QW)) * PG_ROW), 16, 0, 0);
   };
   auto issue = [&](int kt, int s) {
 #pragma unroll
@@ -1615,27 +1630,27 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   };
 
 
-  // fragment rows of this lane: W row wn * 128 + 32 i + l % 32, x row
+  // fragment rows of this lane: W row wn * CPW + 32 i + l % 32, x row
   // wm * TPW + 32 j + l % 32 (both = l % 32 modulo 32, so one swizzle);
   // k chunk 2 kk + l / 32 of the stage
   const int sw = (fr & 7) ^ ((fr >> 3) & 1);
-  auto read_at = [&](int s, int kk, u32x4 (&fa_)[4], u32x4 (&fb_)[NJ], int idx) {
+  auto read_at = [&](int s, int kk, u32x4 (&fa_)[NI], u32x4 (&fb_)[NJ], int idx) {
     const char* st = pg_lds + s * Geo::STAGE + fr * PG_ROW + (((2 * kk + fh) ^ sw) << 4);
-    if (idx < 4)
-      fa_[idx] = *reinterpret_cast<const u32x4*>(st + (wn * 128 + 32 * idx) * PG_ROW);
+    if (idx < NI)
+      fa_[idx] = *reinterpret_cast<const u32x4*>(st + (wn * CPW + 32 * idx) * PG_ROW);
     else
-      fb_[idx - 4] = *reinterpret_cast<const u32x4*>(st + PG_N * PG_ROW + (wm * TPW + 32 * (idx - 4)) * PG_ROW);
+      fb_[idx - NI] = *reinterpret_cast<const u32x4*>(st + NT * PG_ROW + (wm * TPW + 32 * (idx - NI)) * PG_ROW);
   };
 
   // Fragments of the four k-steps of a stage sit in four register sets,
-  // read two k-steps ahead of their MFMAs.  Stage kt + 2 is requested into
-  // slot kt % 2 after the barrier at mid-stage kt that ends every wave's
+  // read two k-steps ahead of their MFMAs.  Stage kt + SLOTS is requested into
+  // slot kt % SLOTS after the barrier at mid-stage kt that ends every wave's
   // reads of it (the fragments of k-steps 2 and 3 were read during k-steps
   // 0 and 1); the same barrier publishes stage kt + 1, whose first two
   // k-steps are read during the last two of stage kt.  The loop has no
   // branches: past the last stage the requests re-read stage nk - 1 into
   // the free slot, which only the discarded reads at the very end look at.
-  u32x4 fa[4][4], fb[4][NJ];
+  u32x4 fa[4][NI], fb[4][NJ];
   // LoRA entries of the segments the tile overlaps, requested ahead of the
   // DMA (so that waiting for them does not wait for it) and put in LDS
   // after it: thread t takes segment sg0 + t
@@ -1658,11 +1673,11 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
       my.scale = *(const __attribute__((address_space(1))) float*)(ep + offsetof(swl_lora_entry, scale));
     }
   }
-  issue(0, 0);
-  issue(min(1, nk - 1), 1);
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) issue(min(i, nk - 1), i);
   build_rowtab();
   if ((int)threadIdx.x < nseg) segl[threadIdx.x] = my;
-  __builtin_amdgcn_s_waitcnt(wait_vm_imm(NREQ));
+  __builtin_amdgcn_s_waitcnt(wait_vm_imm(NREQ * (SLOTS - 1)));
   lds_barrier();
   // The main loop over a predicate live(j): whether the wave's 32-row block
   // j of token rows holds a row of the batch.  Every block does, except in
@@ -1671,7 +1686,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   // costs a fraction of a full one; the DMA requests and barriers stay the
   // same in every wave.
   auto main_loop = [&](auto live) {
-    auto read_live = [&](int idx) { return idx < 4 ? live(0) : live(idx - 4); };
+    auto read_live = [&](int idx) { return idx < NI ? live(0) : live(idx - NI); };
 #pragma unroll
     for (int idx = 0; idx < NR; ++idx)
       if (read_live(idx)) read_at(0, 0, fa[0], fb[0], idx);
@@ -1679,7 +1694,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
     for (int idx = 0; idx < NR; ++idx)
       if (read_live(idx)) read_at(0, 1, fa[1], fb[1], idx);
     for (int kt = 0; kt < nk; ++kt) {
-      const int s = kt & 1;
+      const int s = kt & (SLOTS - 1), s1 = (kt + 1) & (SLOTS - 1);
       // k-steps 0, 1 of stage kt; reads of its k-steps 2, 3 during the first
       // 2 NR
 #pragma unroll
@@ -1692,21 +1707,22 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      // this wave's DMA of stage kt + 1 has landed (it is all that is
-      // outstanding), then every wave's; every wave is past its reads of slot s
-      __builtin_amdgcn_s_waitcnt(wait_vm_imm(0));
+      // this wave's DMA of stage kt + 1 has landed (the later SLOTS - 2 stages
+      // may be outstanding), then every wave's; every wave is past its reads
+      // of slot s
+      __builtin_amdgcn_s_waitcnt(wait_vm_imm(NREQ * (SLOTS - 2)));
       lds_barrier();
       __builtin_amdgcn_sched_barrier(0);
       // k-steps 2, 3; reads of stage kt + 1's k-steps 0, 1 during the first
-      // 2 NR, the NREQ DMA requests of stage kt + 2 spread over the 2 MF MFMAs
-      const int nx = min(kt + 2, nk - 1);
+      // 2 NR, the NREQ DMA requests of stage kt + SLOTS spread over the 2 MF MFMAs
+      const int nx = min(kt + SLOTS, nk - 1);
 #pragma unroll
       for (int t = 0; t < 2 * MF; ++t) {
         if (live(t % NJ)) mfma_at(fa[2], fb[2], fa[3], fb[3], t);
         if (t < NR) {
-          if (read_live(t)) read_at(s ^ 1, 0, fa[0], fb[0], t);
+          if (read_live(t)) read_at(s1, 0, fa[0], fb[0], t);
         } else if (t < 2 * NR) {
-          if (read_live(t - NR)) read_at(s ^ 1, 1, fa[1], fb[1], t - NR);
+          if (read_live(t - NR)) read_at(s1, 1, fa[1], fb[1], t - NR);
         }
         if (t == 0 || (t * NREQ) / (2 * MF) != ((t - 1) * NREQ) / (2 * MF)) request_at(nx, s, (t * NREQ) / (2 * MF));
         __builtin_amdgcn_sched_barrier(0);
@@ -1729,11 +1745,12 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   // bf16 (zero for the other segments' rows), 16 ranks a step.  The steps
   // run as one loop over (segment, rank step) with the next step's loads in
   // flight while the current one's MFMAs issue (two register sets taking
-  // turns), the entries read from the tile's LDS table.
+  // turns), the entries read from the tile's LDS table.  With K split, the
+  // segments are dealt over the splits.
   if (lora_k) {
     const int64_t bstart = blk_start_of(a.L, lb);
-    auto first = [&](int i) {  // first segment from i with an adapter
-      while (i < nseg && segl[i].rank <= 0) ++i;
+    auto first = [&](int i) {  // first segment from i with an adapter (of this split's)
+      while (i < nseg && (segl[i].rank <= 0 || (SPLIT && i % a.n_split != sp))) ++i;
       return i;
     };
     auto advance = [&](int& i, int& q0) {
@@ -1743,12 +1760,12 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
         i = first(i + 1);
       }
     };
-    auto load = [&](int i, int q0, u32x4 (&fa_)[4], u32x4 (&u_)[NJ][2]) {
+    auto load = [&](int i, int q0, u32x4 (&fa_)[NI], u32x4 (&u_)[NJ][2]) {
       const PgSegLora e = segl[i];
       const int r = e.rank, q = q0 + 8 * fh;
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int64_t n = n0 + wn * 128 + 32 * i4 + fr;
+      for (int i4 = 0; i4 < NI; ++i4) {
+        const int64_t n = n0 + wn * CPW + 32 * i4 + fr;
         fa_[i4] = (n < a.N && q < r) ? ld16(e.b + (n - bstart) * r + q) : u32x4{0u, 0u, 0u, 0u};
       }
       const int64_t lo = a.out.off[sg0 + i], hi = a.out.off[sg0 + i + 1];
@@ -1764,7 +1781,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
         }
       }
     };
-    auto use = [&](int i, const u32x4 (&fa_)[4], const u32x4 (&u_)[NJ][2]) {
+    auto use = [&](int i, const u32x4 (&fa_)[NI], const u32x4 (&u_)[NJ][2]) {
       const float scale = segl[i].scale;
       u32x4 fb_[NJ];
 #pragma unroll
@@ -1784,7 +1801,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
     // of the next PD - 1 steps are in flight (a tile over many small
     // segments runs ~20 latency-bound steps)
     constexpr int PD = 3;
-    u32x4 ra[PD][4], ru[PD][NJ][2];
+    u32x4 ra[PD][NI], ru[PD][NJ][2];
     int di[PD];
     int li = first(0), lq = 0;  // the next step to load
 #pragma unroll
@@ -1810,16 +1827,16 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   }
 
   // Epilogue through LDS (the stages are free once every wave is past its
-  // last reads), in two halves of the columns so each wave's share fits:
+  // last reads), 64 of each wave's columns at a time so its share fits:
   // acc[i][j] element e of lane l is column 32 i + 8 (e / 4) + 4 (l / 32) +
-  // e % 4 of the wave's 128, token 32 j + l % 32.  Wave w's half h lands in
+  // e % 4 of the wave's CPW, token 32 j + l % 32.  Wave w's half h lands in
   // region w as [TPW tokens][64 columns (+4 pad)] fp32; then thread t takes
   // quads of four columns, 16 threads a token row, and finishes them
   // (bias, LoRA expand, one bf16 rounding, the segment's row).
   constexpr int ELD = PG_ELD;
   float* reg = reinterpret_cast<float*>(pg_lds) + wv * TPW * ELD;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < NI / 2; ++h) {
     lds_barrier();  // the previous half's (or the k-loop's) reads are done
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii)
@@ -1832,7 +1849,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
           *reinterpret_cast<f32x4*>(reg + tok * ELD + col) = f32x4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
         }
     lds_barrier();
-    // items: wave region w2 (tokens wm2 * TPW, columns wn2 * 128 + 64 h),
+    // items: wave region w2 (tokens wm2 * TPW, columns wn2 * CPW + 64 h),
     // token row tr, quad cq; WAVES x TPW x 16 items, 8 NJ a thread (row
     // group t / 16 of RG, rows rg + RG kk of each region), all of one
     // thread's in the two column quads cq = t % 16 of the two wn2, whose
@@ -1842,15 +1859,15 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
     float bq[2][4];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const int64_t n = n0 + c * 128 + 64 * h + 4 * cq;
+      const int64_t n = n0 + c * CPW + 64 * h + 4 * cq;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bq[c][e] = (a.bias && n + e < a.N) ? bf2f(a.bias[n + e]) : 0.f;
+      for (int e = 0; e < 4; ++e) bq[c][e] = (a.bias && !(SPLIT && a.part) && n + e < a.N) ? bf2f(a.bias[n + e]) : 0.f;
     }
     auto item = [&](int k, bool lora) {
       const int w2 = k / KK, tr = (threadIdx.x >> 4) + RG * (k % KK);
       const int row = (w2 >> 1) * TPW + tr;
       const int64_t m = m0 + row;
-      const int64_t n = n0 + (w2 & 1) * 128 + 64 * h + 4 * cq;
+      const int64_t n = n0 + (w2 & 1) * CPW + 64 * h + 4 * cq;
       if (m >= a.M || n >= a.N) return;
       const f32x4 q4 = *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(pg_lds) + (w2 * TPW + tr) * ELD + 4 * cq);
       float v[4];
@@ -1858,9 +1875,26 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
       for (int e = 0; e < 4; ++e) v[e] = q4[e] + bq[w2 & 1][e];
       epilogue_store4(v, n, a.N, nullptr, a.L, lora ? lidxtab[row] : -1, (int)m, rowtab[row]);
     };
-    if (a.has_lora && !a.lora_mfma) {
+    if (SPLIT && a.part) {  // this split's fp32 tile
+#pragma unroll
+      for (int w2 = 0; w2 < WAVES; ++w2)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+          const int tr = (threadIdx.x >> 4) + RG * kk;
+          const f32x4 q = *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(pg_lds) + (w2 * TPW + tr) * ELD + 4 * cq);
+          const int64_t m = m0 + (w2 >> 1) * TPW + tr, n = n0 + (w2 & 1) * CPW + 64 * h + 4 * cq;
+          float* dst = a.part + ((int64_t)sp * (a.M - a.m_base) + m - a.m_base) * a.N + n;
+          if (m >= a.M || n >= a.N) continue;
+          if ((a.N & 3) == 0) {
+            *(__attribute__((address_space(1))) f32x4*)(dst) = q;
+          } else {
+            for (int e = 0; e < 4; ++e)
+              if (n + e < a.N) dst[e] = q[e];
+          }
+        }
+    } else if (a.has_lora && !a.lora_mfma) {
       // the LoRA delta in the epilogue (per-quad loads of u and lora_B)
-      for (int k = 0; k < 8 * NJ; ++k) item(k, true);
+      for (int k = 0; k < WAVES * KK; ++k) item(k, true);
     } else {
       // k = KK w2 + kk: the KK staged quads and row pointers of a region
       // are read together, then stored
@@ -1874,7 +1908,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
           q[kk] = *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(pg_lds) + (w2 * TPW + tr) * ELD + 4 * cq);
           rp[kk] = rowtab[(w2 >> 1) * TPW + tr];
         }
-        const int64_t n = n0 + (w2 & 1) * 128 + 64 * h + 4 * cq;
+        const int64_t n = n0 + (w2 & 1) * CPW + 64 * h + 4 * cq;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
           const int64_t m = m0 + (w2 >> 1) * TPW + (threadIdx.x >> 4) + RG * kk;
@@ -1888,6 +1922,40 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
       }
     }
   }
+}
+
+// The split prefill GEMM's output: the splits' fp32 tiles summed in order,
+// bias (and the LoRA delta where the tiles could not carry it), one rounding,
+// the row's slot.  One thread per 4 columns of a row.
+__global__ __launch_bounds__(256) void prefill_fold_kernel(TiledArgs a) {
+  const int64_t m = a.m_base + blockIdx.y;
+  const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (n >= a.N) return;
+  const int sg = a.y ? 0 : find_seg(a.out.off, a.out.n, m);
+  bf16* yrow = a.y ? a.y + m * a.ldy
+                   : reinterpret_cast<bf16*>(const_cast<void*>(a.out.ptr[sg])) + (m - a.out.off[sg]) * a.N;
+  const float* p = a.part + (int64_t)blockIdx.y * a.N + n;
+  const int64_t stride = (a.M - a.m_base) * a.N;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < a.n_split; k0 += 4) {
+    f32x4 q[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      q[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (k0 + k >= a.n_split) continue;
+      if ((a.N & 3) == 0) {
+        q[k] = *(const __attribute__((address_space(1))) f32x4*)(p + (k0 + k) * stride);
+      } else {
+        for (int e = 0; e < 4; ++e)
+          if (n + e < a.N) q[k][e] = p[(k0 + k) * stride + e];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += q[k][e];
+  }
+  epilogue_store4(v, n, a.N, a.bias, a.L, a.has_lora && !a.lora_mfma ? a.seg_lora[sg] : -1, (int)m, yrow);
 }
 
 // ----------------------------------------------- generic small matmul -----
@@ -4149,6 +4217,18 @@ int scratch_get(size_t need, hipStream_t stream, void** out) {
   return SWL_OK;
 }
 
+// Whether scratch_get would give `need` bytes: it has them, or may grow.
+bool scratch_may_hold(size_t need, hipStream_t stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  {
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    if (dev < (int)g_scratch.size() && g_scratch[dev].bytes >= need) return true;
+  }
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return !stream || (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone);
+}
+
 // ---------------------------------------------------------- launch timer
 // Optional HIP-event timing of the decode projection: when armed, every
 // launch_skinny call (outside graph capture) launches its base kernel and
@@ -4716,49 +4796,14 @@ int launch_skinny(const bf16* w, const bf16* bias, int64_t N, int64_t K, int nto
 // multiple of the 256 x 256 kernel's 64-wide stages.
 bool prefill_uses_tiled(int64_t K) { return K % PG_K != 0 || K < PG_K; }
 
-template <int NJ, int WM>
-int launch_gemm256(const TiledArgs& a, int tiles_m, int tiles, int per_xcd, int gm, hipStream_t st) {
-  constexpr size_t lds = PgGeom<NJ, WM>::LDS;
+template <int NI, int NJ, int WM, int SLOTS>
+int launch_gemm256(const TiledArgs& a, hipStream_t st) {
+  using Geo = PgGeom<NI, NJ, WM, SLOTS>;
   static size_t allowed = 0;
-  int rc = allow_lds(gemm256_kernel<NJ, WM>, lds, &allowed);
+  int rc = allow_lds(gemm256_kernel<NI, NJ, WM, SLOTS>, Geo::LDS, &allowed);
   if (rc) return rc;
-  hipLaunchKernelGGL((gemm256_kernel<NJ, WM>), dim3((unsigned)(8 * per_xcd)), dim3(128 * WM), lds, st, a, tiles_m,
-                     tiles, per_xcd, gm);
-  return SWL_OK;
-}
-
-int launch_prefill_gemm(const TiledArgs& a, hipStream_t st) {
-  if (prefill_uses_tiled(a.K)) {
-    const dim3 grid((unsigned)((a.N + TN - 1) / TN), (unsigned)((a.M + TM - 1) / TM));
-    hipLaunchKernelGGL(tiled_kernel, grid, dim3(256), 0, st, a);
-    SWL_LAUNCH_CHECK("tiled_kernel launch");
-    return SWL_OK;
-  }
-  // token rows a tile: 256, or 192 where the grid then covers the CUs in
-  // fewer tile times (a 192-row tile measured at ~0.9 of a 256-row one: the
-  // W side streams the same bytes): the O and Down rounds at 2325 rows have
-  // 160 tiles of 256 for 256 CUs, 208 of 192 (146 -> 133 us, 370 -> 335).
-  // A tile of the last row tile costs the share of its first row wave's
-  // 32-row blocks that hold rows, at least 0.4 of a full tile (its stages
-  // still wait for their DMA); such tiles first fill the CUs the last wave
-  // of full tiles leaves idle.
-  const int tiles_n = (int)((a.N + PG_N - 1) / PG_N);
-  const int64_t cus = cu_count();
-  auto cost = [&](int nj) {
-    const int64_t mt = 64 * nj, full = (a.M / mt) * tiles_n, rem = a.M % mt;
-    const double pc = rem ? std::max(0.4, (double)std::min<int64_t>(nj, (rem + 31) / 32) / nj) : 0.0;
-    const int64_t waves = (full + cus - 1) / cus;
-    const double spill = (rem ? pc * tiles_n : 0.0) - (double)(waves * cus - full);
-    const double t = (double)waves + (spill > 0 ? std::ceil(spill / ((double)cus * pc)) * pc : 0.0);
-    return t * (nj == 3 ? 0.9 : 1.0);
-  };
-  static const int forced = [] {
-    const char* e = getenv("SWL_PREFILL_NJ");
-    return e ? atoi(e) : 0;
-  }();
-  const int nj = (forced == 3 || forced == 4) ? forced : (cost(3) < cost(4) ? 3 : 4);
-  const int tiles_m = (int)((a.M + 64 * nj - 1) / (64 * nj));
-  const int tiles = tiles_m * tiles_n;
+  const int tiles_m = (int)((a.M - a.m_base + Geo::MT - 1) / Geo::MT);
+  const int tiles = tiles_m * (int)((a.N + Geo::NT - 1) / Geo::NT);
   const int per_xcd = (tiles + 7) / 8;
   // Tile order.  Every XCD (workgroup i on XCD i % 8) walks a contiguous run
   // of per_xcd linear tiles.  When all tiles run at once (no more tiles than
@@ -4767,11 +4812,114 @@ int launch_prefill_gemm(const TiledArgs& a, hipStream_t st) {
   // fewer distinct W and row slices than with all row tiles of a column
   // fastest.  Rounds of several waves keep the rows fastest (one group).
   int gm = tiles_m;
-  if (tiles <= cus) gm = std::max(1, std::min(tiles_m, (int)std::lround(std::sqrt((double)per_xcd))));
-  const int rc = nj == 3 ? launch_gemm256<3, 2>(a, tiles_m, tiles, per_xcd, gm, st)
-                          : launch_gemm256<4, 2>(a, tiles_m, tiles, per_xcd, gm, st);
-  if (rc) return rc;
+  if (tiles <= cu_count()) gm = std::max(1, std::min(tiles_m, (int)std::lround(std::sqrt((double)per_xcd))));
+  hipLaunchKernelGGL((gemm256_kernel<NI, NJ, WM, SLOTS>), dim3((unsigned)(8 * per_xcd), (unsigned)a.n_split),
+                     dim3(128 * WM), Geo::LDS, st, a, tiles_m, tiles, per_xcd, gm);
   SWL_LAUNCH_CHECK("gemm256_kernel launch");
+  return SWL_OK;
+}
+
+// Tile of a prefill GEMM (nj: 4 = 256 x 256, 3 = 256 x 192, 2 = 128 x 128) and
+// the K splits of the last, by estimated time; `split_ok`: the caller has
+// scratch for the splits' fp32 tiles.  The 128 x 128 tile runs at 0.7 of the
+// large ones' rate once they fill the chip, but a short batch leaves most CUs
+// without a large tile: measured per round with rank-16 adapters, large ->
+// 128 x 128 (us), 107 rows: QKV 104 -> 34, O 102 -> 31, Gate+Up 87 -> 54, Down
+// 305 -> 53; 512 rows: 97 -> 55, 94 -> 44, 134 -> 176 (kept large), 281 -> 97;
+// 1000 rows: 98 -> 96, 94 -> 55, 259 -> 323 (large), 274 -> 154; level or
+// large from ~1500 rows.
+// Rows that would start another wave of large tiles go to 128 x 128 tiles
+// behind them: 2997 rows, QKV: 16 x 24 tiles of 192 rows, 1.5 waves; 10 x 24
+// of 256 rows, then 437 rows in 128 x 128 tiles (201 -> 164 us).
+struct PrefillPlan {
+  int nj = 4;           // of the rows before `rows`
+  int64_t rows = 0;     // in large tiles; the rest in 128 x 128 tiles
+  int n_split = 1;
+};
+PrefillPlan plan_prefill(int64_t M, int64_t N, int64_t K, bool split_ok) {
+  PrefillPlan p;
+  static const int forced = [] {
+    const char* e = getenv("SWL_PREFILL_NJ");
+    return e ? atoi(e) : 0;
+  }();
+  const int64_t cus = cu_count(), stages = K / PG_K;
+  // Large tiles, in tile times: 256 token rows, or 192 where the grid then
+  // covers the CUs in fewer of them (a 192-row tile measured at ~0.9 of a
+  // 256-row one: the W side streams the same bytes): the O and Down rounds at
+  // 2325 rows have 160 tiles of 256 for 256 CUs, 208 of 192 (146 -> 133 us,
+  // 370 -> 335).  A tile of the last row tile costs the share of its first row
+  // wave's 32-row blocks that hold rows, at least 0.4 of a full tile (its
+  // stages still wait for their DMA); such tiles first fill the CUs the last
+  // wave of full tiles leaves idle, and where they do not fit there they
+  // start another.
+  const int64_t tiles_n = (N + PG_N - 1) / PG_N;
+  auto cost = [&](int nj) {
+    const int64_t mt = 64 * nj, full = (M / mt) * tiles_n, rem = M % mt;
+    const double pc = rem ? std::max(0.4, (double)std::min<int64_t>(nj, (rem + 31) / 32) / nj) : 0.0;
+    const int64_t waves = (full + cus - 1) / cus;
+    const int64_t spill = (rem ? tiles_n : 0) - (waves * cus - full);
+    const double t = (double)waves + (spill > 0 ? (double)((spill + cus - 1) / cus) * pc : 0.0);
+    return t * (nj == 3 ? 0.9 : 1.0);
+  };
+  p.nj = forced == 3 || forced == 4 ? forced : cost(3) < cost(4) ? 3 : 4;
+  p.rows = M;
+  if (forced == 3 || forced == 4) return p;
+  // us: a large tile's stage takes 1.25 with few CUs busy, 1.85 with all (the
+  // clock falls with the load); a 128 x 128 stage 0.65, the splits' sum a
+  // launch (5) and their bytes, written and read, at 4 TB/s; a second launch 8
+  // (the first one's last tiles, and its own ramp)
+  auto large = [&](int nj, int64_t rows, double waves) {
+    const int64_t tiles = (rows + 64 * nj - 1) / (64 * nj) * tiles_n;
+    return waves * (double)stages * (1.25 + 0.6 * std::min(1.0, (double)tiles / (double)cus));
+  };
+  auto small = [&](int64_t rows, int s) {
+    const int64_t tiles = (rows + 127) / 128 * ((N + 127) / 128);
+    return (double)((tiles * s + cus - 1) / cus) * (double)((stages + s - 1) / s) * 0.65 +
+           (s > 1 ? 5.0 + (double)(s * rows * N) * 8.0 / 4e6 : 0.0);
+  };
+  const int most = split_ok ? (int)std::max<int64_t>(1, std::min<int64_t>(16, stages / 4)) : 1;
+  double best = forced == 2 ? 1e30 : large(p.nj, M, cost(p.nj));
+  auto take = [&](double t, int nj, int64_t rows, int s) {
+    if (t < best) {
+      best = t;
+      p.nj = nj;
+      p.rows = rows;
+      p.n_split = s;
+    }
+  };
+  for (int s = 1; s <= most; ++s) take(small(M, s), 4, 0, s);
+  if (forced == 2) return p;
+  for (int nj = 3; nj <= 4; ++nj)
+    for (int64_t rows = 64 * nj; rows < M; rows += 64 * nj) {
+      const double t = large(nj, rows, (double)((rows / (64 * nj) * tiles_n + cus - 1) / cus) * (nj == 3 ? 0.9 : 1.0)) + 8.0;
+      if (t >= best) break;
+      for (int s = 1; s <= most; ++s) take(t + small(M - rows, s), nj, rows, s);
+    }
+  return p;
+}
+
+int launch_prefill_gemm(TiledArgs a, const PrefillPlan& p, hipStream_t st) {
+  a.n_split = 1;
+  if (prefill_uses_tiled(a.K)) {
+    const dim3 grid((unsigned)((a.N + TN - 1) / TN), (unsigned)((a.M + TM - 1) / TM));
+    hipLaunchKernelGGL(tiled_kernel, grid, dim3(256), 0, st, a);
+    SWL_LAUNCH_CHECK("tiled_kernel launch");
+    return SWL_OK;
+  }
+  if (p.rows > 0) {
+    TiledArgs b = a;
+    b.M = std::min(a.M, p.rows);
+    b.part = nullptr;
+    int rc = p.nj == 3 ? launch_gemm256<4, 3, 2, 2>(b, st) : launch_gemm256<4, 4, 2, 2>(b, st);
+    if (rc || p.rows >= a.M) return rc;
+  }
+  a.m_base = p.rows;
+  if (a.part) a.n_split = p.n_split;
+  int rc = launch_gemm256<2, 2, 2, 4>(a, st);
+  if (rc || !a.part) return rc;
+  hipLaunchKernelGGL(prefill_fold_kernel, dim3((unsigned)((a.N + 1023) / 1024), (unsigned)(a.M - a.m_base)),
+                     dim3(256), 0, st, a);
+  SWL_LAUNCH_CHECK("prefill_fold_kernel launch");
   return SWL_OK;
 }
 
@@ -5112,7 +5260,7 @@ int swl_gemm_bf16(const void* x, const void* w, const void* bias, void* y, int64
   a.y = reinterpret_cast<bf16*>(y);
   a.ldy = n;
   a.has_lora = 0;
-  return launch_prefill_gemm(a, st);
+  return launch_prefill_gemm(a, plan_prefill(m, n, k, false), st);
 }
 
 int swl_round_bf16(int n_seg, const int64_t* rows, const void* const* seg_in, void* const* seg_out, const void* w,
@@ -6129,8 +6277,19 @@ int round_launch_ws(int n_seg, const int64_t* rows, const void* const* seg_in, v
   }
   size_t ubytes = 0;
   if (has_lora) ubytes = sizeof(float) * (size_t)u_ks * (size_t)T * (size_t)u_ld;
+  // K splits only where the round takes scratch anyway (its LoRA shrink): a
+  // round without adapters stays free of it, so such rounds on several
+  // streams stay independent; and not where a captured round would need more
+  // of it than there is
+  const size_t ubytes_al = (ubytes + 255) & ~(size_t)255;
+  PrefillPlan plan = plan_prefill(T, N, K, has_lora && !packed_x && T <= 65535);
+  size_t pbytes = plan.n_split > 1 ? sizeof(float) * (size_t)plan.n_split * (size_t)(T - plan.rows) * (size_t)N : 0;
+  if (pbytes && !scratch_may_hold(xbytes_al + ubytes_al + pbytes, st)) {
+    plan.n_split = 1;
+    pbytes = 0;
+  }
   void* scr = nullptr;
-  int rc = scratch_get(xbytes_al + ubytes, st, &scr);
+  int rc = scratch_get(xbytes_al + (pbytes ? ubytes_al + pbytes : ubytes), st, &scr);
   if (rc) return rc;
   bf16* packed = reinterpret_cast<bf16*>(scr);
   if (packed_x) {
@@ -6171,14 +6330,15 @@ int round_launch_ws(int n_seg, const int64_t* rows, const void* const* seg_in, v
     // the 256 x 256 kernel adds the LoRA delta as MFMA k-steps when every
     // tile lies inside one column block and the ranks are multiples of 8
     a.lora_mfma = 1;
-    for (int b = 1; b < nblk; ++b) a.lora_mfma &= (L.blk_start[b] % PG_N == 0) ? 1 : 0;
+    for (int b = 1; b < nblk; ++b) a.lora_mfma &= (L.blk_start[b] % (plan.rows == 0 ? 128 : PG_N) == 0) ? 1 : 0;
     for (int i = 0; i < n_seg; ++i)
       if (a.seg_lora[i] >= 0) {
         const int r = host_entries[a.seg_lora[i]].rank;
         a.lora_mfma &= (r % 8 == 0 && r <= 64) ? 1 : 0;
       }
   }
-  return launch_prefill_gemm(a, st);
+  if (pbytes) a.part = reinterpret_cast<float*>(reinterpret_cast<char*>(scr) + xbytes_al + ubytes_al);
+  return launch_prefill_gemm(a, plan, st);
 }
 
 }  // namespace swl

@@ -1,0 +1,100 @@
+"""GPU tests of the prefill round just past the decode regime: 128 x 128 tiles
+with and without K splits, their edges and remainders, LoRA carried by the
+tiles, by the splits' sum and by the large tiles' epilogue, against float32
+products of the same bf16 operands (bound: the result's bf16 rounding, 1e-2 of
+the largest output as everywhere)."""
+
+import pytest
+import torch
+
+from tests._util import BF16, assert_close, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _round(dev, rows, n, k, cols, ranks, bias=False, seed=0):
+    """One round over `rows`, segment i with an adapter of ranks[i] (0: none)
+    -> (outputs, expected)."""
+    from swarmlora_amd import ops
+    w = randn((n, k), seed, std=0.02).to(dev)
+    b = randn((n,), seed + 1).to(dev) if bias else None
+    xs = [randn((r, k), seed + 2 + i).to(dev) for i, r in enumerate(rows)]
+    # sentinel rows after each slot's rows
+    bufs = [torch.full((r + 1, n), 9.0, dtype=BF16, device=dev) for r in rows]
+    table, ids, want = ops.LoraTable(dev), [], []
+    for i, (x, r) in enumerate(zip(xs, ranks)):
+        y = x.float() @ w.float().t() + (b.float() if bias else 0)
+        if r:
+            a = randn((r * len(cols), k), 50 + i, std=0.02).to(dev)
+            bs = [randn((c, r), 80 + 7 * i + j, std=0.02).to(dev) for j, c in enumerate(cols)]
+            u = x.float() @ a.float().t()
+            y += 2.0 * torch.cat([u[:, j * r:(j + 1) * r] @ bs[j].float().t() for j in range(len(cols))], 1)
+            ids.append(table.add(a, bs, r, 2.0))
+        else:
+            ids.append(-1)
+        want.append(y)
+    lora = any(ranks)
+    ops.round_fused(xs, bufs, rows, w, b, seg_lora=ids if lora else None, table=table if lora else None,
+                    blk_cols=cols if lora else None)
+    torch.cuda.synchronize()
+    for o in bufs:
+        assert bool((o[-1] == 9.0).all())
+    return [o[:-1] for o in bufs], want
+
+
+@pytest.mark.parametrize("rows,n,k,cols,ranks,bias", [
+    ([65], 128, 64, [128], [16], True),                              # one tile, one stage
+    ([1, 64], 256, 2048, [128, 128], [8, 64], False),                # splits of 4 stages and more
+    ([100, 3, 26], 1536, 4096, [1024, 256, 256], [16, 0, 32], True),  # a full row tile and one row
+    ([128], 384, 8192, [384], [24], False),
+    ([90, 40], 200, 4096, [72, 128], [16, 16], True),                # blocks not on tile bounds: delta in the sum
+    ([70], 130, 2048, [130], [12], False),                           # ... rank not a multiple of 8, n % 4
+    ([300, 1, 1, 1], 2048, 1024, [2048], [16, 8, 0, 64], False),
+    ([66, 62], 1000, 4160, [1000], [0, 0], True),                    # no adapters: no splits
+])
+def test_short_prefill_rounds(dev, rows, n, k, cols, ranks, bias):
+    got, want = _round(dev, rows, n, k, cols, ranks, bias)
+    for g, w in zip(got, want):
+        assert_close(g, w, what=f"{rows} {n} {k}")
+
+
+def test_short_prefill_round_captured_without_room_for_splits(dev):
+    """A captured round that would need more scratch for its splits than the
+    library holds runs unsplit (its shrink fits what an earlier call sized),
+    and replays give the eager result."""
+    import subprocess
+    import sys
+    code = """
+import torch
+from swarmlora_amd import ops
+bf = torch.bfloat16
+g = torch.Generator(device="cuda").manual_seed(3)
+rn = lambda *s: torch.randn(*s, generator=g, device="cuda").to(bf)
+def call(n, k, rows):
+    t = ops.LoraTable("cuda")
+    t.add(rn(16, k) * 0.05, [rn(n, 16) * 0.05], 16, 2.0)
+    x, y, w = rn(rows, k), torch.zeros(rows, n, dtype=bf, device="cuda"), rn(n, k) * 0.05
+    t.device_table()
+    return y, lambda: ops.round_fused([x], [y], [rows], w, None, [0], t, [n])
+_, small = call(256, 512, 70)   # sizes the scratch: its smallest step
+small()
+torch.cuda.synchronize()
+y, big = call(4096, 4096, 128)  # its splits would need 16 MB
+gr = torch.cuda.CUDAGraph()
+with torch.cuda.graph(gr):
+    big()
+outs = []
+for _ in range(3):
+    y.zero_()
+    gr.replay()
+    torch.cuda.synchronize()
+    outs.append(y.clone())
+assert all(torch.equal(o, outs[0]) for o in outs)
+big()
+torch.cuda.synchronize()
+d = (y.float() - outs[0].float()).abs().max() / y.float().abs().max()
+assert float(d) < 1e-2, float(d)
+print("captured ok")
+"""
+    p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0 and "captured ok" in p.stdout, p.stdout + p.stderr
