@@ -18,9 +18,11 @@
 //                           the LoRA expand u . B^T * scale, rounds once and
 //                           stores each token's row into its slot buffer (the
 //                           scatter is fused).
-//   gemm256_kernel          M > 64 "prefill" projection: 256x256 (or 256x192)
-//                           MFMA tiles fed by LDS-DMA, rows read in place from
-//                           the slot buffers, the LoRA delta as extra k-steps.
+//   gemm256_kernel          M > 64 "prefill" projection: 256x256 (256x192,
+//                           128x128 for short rounds) MFMA tiles fed by
+//                           LDS-DMA, rows read in place from the slot buffers,
+//                           the LoRA delta as extra k-steps; 128 columns by 32
+//                           or 64 rows for a row-major LM head.
 //   tiled_kernel            the prefill projection for K not a multiple of 64:
 //                           128x128x64 LDS-staged MFMA tiles over a gathered
 //                           copy, fp32 accumulation, same epilogue.
@@ -1504,7 +1506,8 @@ __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
                                                  0, 0, 0);
 }
 
-template <int NI, int NJ, int WM, int SLOTS>
+// WNT: W read non-temporal (a batch of one row tile reads it once).
+template <int NI, int NJ, int WM, int SLOTS, bool WNT = false>
 __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int tiles_m, int tiles, int per_xcd,
                                                                int gm) {
   // SLOTS x [W NT x 64 | x MT x 64]; then the epilogue's WAVES x [TPW][PG_ELD] fp32
@@ -1515,8 +1518,10 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   constexpr int WR = NT / WAVES;                                // W rows a wave moves per stage
   constexpr int MF = NI * NJ, NR = NI + NJ;                     // MFMAs and fragment reads per k-step
   constexpr int NREQ = WR / 8 + XR / 8;                         // DMA instructions a wave per stage
-  static_assert(WR % 16 == 0 && XR % 16 == 0 && NR <= MF, "the waves' DMA rows must cover the stage");
-  static_assert((SLOTS & (SLOTS - 1)) == 0 && NREQ * (SLOTS - 1) < 64, "slots are a power of two");
+  static_assert(WR % 16 == 0 && XR % 16 == 0, "the waves' DMA rows must cover the stage");
+  static_assert(SLOTS >= 2 && NREQ * (SLOTS - 1) < 64, "the stages in flight must fit the counter");
+  constexpr bool POW2 = (SLOTS & (SLOTS - 1)) == 0;
+  constexpr int RPM = (NR + MF - 1) / MF;  // fragment reads per MFMA
   extern __shared__ __attribute__((aligned(16))) char pg_lds[];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1619,7 +1624,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
     constexpr int QW = WR / 8;
     if (q < QW)
       __builtin_amdgcn_global_load_lds((gbl_ptr)(wsrc[q] + (int64_t)kt * PG_K),
-                                       (lds_ptr)(st + (WR * wv + 8 * q) * PG_ROW), 16, 0, 0);
+                                       (lds_ptr)(st + (WR * wv + 8 * q) * PG_ROW), 16, 0, WNT ? kLoadNT : 0);
     else
       __builtin_amdgcn_global_load_lds((gbl_ptr)(xsrc[q - QW] + (int64_t)kt * PG_K),
                                        (lds_ptr)(st + NT * PG_ROW + (XR * wv + 8 * (q - QW)) * PG_ROW), 16, 0, 0);
@@ -1693,17 +1698,23 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
 #pragma unroll
     for (int idx = 0; idx < NR; ++idx)
       if (read_live(idx)) read_at(0, 1, fa[1], fb[1], idx);
+    int slot = 0;
     for (int kt = 0; kt < nk; ++kt) {
-      const int s = kt & (SLOTS - 1), s1 = (kt + 1) & (SLOTS - 1);
+      const int s = POW2 ? kt & (SLOTS - 1) : slot;
+      const int s1 = POW2 ? (kt + 1) & (SLOTS - 1) : (slot + 1 < SLOTS ? slot + 1 : 0);
+      slot = s1;
       // k-steps 0, 1 of stage kt; reads of its k-steps 2, 3 during the first
       // 2 NR
 #pragma unroll
       for (int t = 0; t < 2 * MF; ++t) {
         if (live(t % NJ)) mfma_at(fa[0], fb[0], fa[1], fb[1], t);
-        if (t < NR) {
-          if (read_live(t)) read_at(s, 2, fa[2], fb[2], t);
-        } else if (t < 2 * NR) {
-          if (read_live(t - NR)) read_at(s, 3, fa[3], fb[3], t - NR);
+#pragma unroll
+        for (int r = RPM * t; r < RPM * (t + 1); ++r) {
+          if (r < NR) {
+            if (read_live(r)) read_at(s, 2, fa[2], fb[2], r);
+          } else if (r < 2 * NR) {
+            if (read_live(r - NR)) read_at(s, 3, fa[3], fb[3], r - NR);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -1719,12 +1730,20 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
 #pragma unroll
       for (int t = 0; t < 2 * MF; ++t) {
         if (live(t % NJ)) mfma_at(fa[2], fb[2], fa[3], fb[3], t);
-        if (t < NR) {
-          if (read_live(t)) read_at(s1, 0, fa[0], fb[0], t);
-        } else if (t < 2 * NR) {
-          if (read_live(t - NR)) read_at(s1, 1, fa[1], fb[1], t - NR);
+#pragma unroll
+        for (int r = RPM * t; r < RPM * (t + 1); ++r) {
+          if (r < NR) {
+            if (read_live(r)) read_at(s1, 0, fa[0], fb[0], r);
+          } else if (r < 2 * NR) {
+            if (read_live(r - NR)) read_at(s1, 1, fa[1], fb[1], r - NR);
+          }
         }
-        if (t == 0 || (t * NREQ) / (2 * MF) != ((t - 1) * NREQ) / (2 * MF)) request_at(nx, s, (t * NREQ) / (2 * MF));
+        if constexpr (NREQ <= 2 * MF) {
+          if (t == 0 || (t * NREQ) / (2 * MF) != ((t - 1) * NREQ) / (2 * MF)) request_at(nx, s, (t * NREQ) / (2 * MF));
+        } else {
+#pragma unroll
+          for (int q = t * NREQ / (2 * MF); q < (t + 1) * NREQ / (2 * MF); ++q) request_at(nx, s, q);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -4796,11 +4815,11 @@ int launch_skinny(const bf16* w, const bf16* bias, int64_t N, int64_t K, int nto
 // multiple of the 256 x 256 kernel's 64-wide stages.
 bool prefill_uses_tiled(int64_t K) { return K % PG_K != 0 || K < PG_K; }
 
-template <int NI, int NJ, int WM, int SLOTS>
-int launch_gemm256(const TiledArgs& a, hipStream_t st) {
+template <int NI, int NJ, int WM, int SLOTS, bool WNT = false>
+int launch_gemm256(const TiledArgs& a, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   using Geo = PgGeom<NI, NJ, WM, SLOTS>;
   static size_t allowed = 0;
-  int rc = allow_lds(gemm256_kernel<NI, NJ, WM, SLOTS>, Geo::LDS, &allowed);
+  int rc = allow_lds(gemm256_kernel<NI, NJ, WM, SLOTS, WNT>, Geo::LDS, &allowed);
   if (rc) return rc;
   const int tiles_m = (int)((a.M - a.m_base + Geo::MT - 1) / Geo::MT);
   const int tiles = tiles_m * (int)((a.N + Geo::NT - 1) / Geo::NT);
@@ -4813,8 +4832,8 @@ int launch_gemm256(const TiledArgs& a, hipStream_t st) {
   // fastest.  Rounds of several waves keep the rows fastest (one group).
   int gm = tiles_m;
   if (tiles <= cu_count()) gm = std::max(1, std::min(tiles_m, (int)std::lround(std::sqrt((double)per_xcd))));
-  hipLaunchKernelGGL((gemm256_kernel<NI, NJ, WM, SLOTS>), dim3((unsigned)(8 * per_xcd), (unsigned)a.n_split),
-                     dim3(128 * WM), Geo::LDS, st, a, tiles_m, tiles, per_xcd, gm);
+  launch_maybe_timed(gemm256_kernel<NI, NJ, WM, SLOTS, WNT>, dim3((unsigned)(8 * per_xcd), (unsigned)a.n_split),
+                     dim3(128 * WM), Geo::LDS, st, e0, e1, a, tiles_m, tiles, per_xcd, gm);
   SWL_LAUNCH_CHECK("gemm256_kernel launch");
   return SWL_OK;
 }
@@ -4915,11 +4934,49 @@ int launch_prefill_gemm(TiledArgs a, const PrefillPlan& p, hipStream_t st) {
   }
   a.m_base = p.rows;
   if (a.part) a.n_split = p.n_split;
-  int rc = launch_gemm256<2, 2, 2, 4>(a, st);
+  int rc = a.M - a.m_base <= 128 ? launch_gemm256<2, 2, 2, 4, true>(a, st) : launch_gemm256<2, 2, 2, 4>(a, st);
   if (rc || !a.part) return rc;
   hipLaunchKernelGGL(prefill_fold_kernel, dim3((unsigned)((a.N + 1023) / 1024), (unsigned)(a.M - a.m_base)),
                      dim3(256), 0, st, a);
   SWL_LAUNCH_CHECK("prefill_fold_kernel launch");
+  return SWL_OK;
+}
+
+// A decode-shaped product with so many columns (an LM head) that 128-column
+// tiles of 32 or 64 token rows fill the chip by themselves: W streamed through
+// LDS once, K whole, the rows stored straight from the tile.  Bound by the read
+// of W; the K-sliced kernel writes and reads fp32 partials on top of it (28
+// rows of 128256: 29 MB each way, and an epilogue launch).  Two workgroups of
+// two waves a CU, three 20 or 24 KiB stages each.  128256 x 4096 (1.05 GB): 28
+// rows 252 -> 166 us (6.3 TB/s), 64 rows 309 -> 186, one row 198 -> 160.
+// Where the line lies (us, sliced -> this): from 16 rows the partials cost more
+// than the tiles that a last wave leaves idle once there are 3/4 of a tile a CU
+// (16 rows of 28672 x 4096: 53.5 -> 51.2, 36864: 68.6 -> 68.7, 64 rows 71 ->
+// 54; half a tile a CU, 16384 x 4096, 16 rows: 34.5 -> 35.7).  Below 16 rows
+// the partials are small, and only a W of 1 GB makes enough waves of tiles (one
+// row of 152064 x 3584: 216 -> 172; 98304 x 4096: 145 -> 149; 65536 x 4096: 98
+// -> 109).
+bool wide_gemm_fits(int64_t m, int64_t n, int64_t k) {
+  if (m > kSkinnyMaxTok || k % PG_K != 0 || prefill_uses_tiled(k)) return false;
+  return m >= 16 ? 4 * ((n + 127) / 128) >= 3 * (int64_t)cu_count() : n * k >= 500000000;
+}
+int launch_wide_gemm(TiledArgs a, hipStream_t st) {
+  a.n_split = 1;
+  const int tslot = timer_slot(st);
+  if (tslot >= 0) {
+    g_timer.N[tslot] = a.N;
+    g_timer.K[tslot] = a.K;
+    g_timer.ntok[tslot] = (int32_t)a.M;
+    g_timer.bytes[tslot] = 2 * (a.N * a.K + a.M * a.K);
+  }
+  hipEvent_t e0 = timer_event(tslot, 0), e1 = timer_event(tslot, 1);
+  int rc = a.M <= 32 ? launch_gemm256<2, 1, 1, 3, true>(a, st, e0, e1) : launch_gemm256<2, 2, 1, 3, true>(a, st, e0, e1);
+  if (rc) return rc;
+  if (tslot >= 0) {
+    // no epilogue kernel: its events mark an empty interval after the product
+    SWL_HIP(hipEventRecord(timer_event(tslot, 2), st));
+    SWL_HIP(hipEventRecord(timer_event(tslot, 3), st));
+  }
   return SWL_OK;
 }
 
@@ -5239,6 +5296,18 @@ int swl_gemm_bf16(const void* x, const void* w, const void* bias, void* y, int64
             SWL_ERR_INVALID, "swl_gemm_bf16: x and w must be 16-byte aligned");
   if (m == 0) return SWL_OK;
   hipStream_t st = (hipStream_t)stream;
+  if (wide_gemm_fits(m, n, k)) {
+    TiledArgs a{};
+    a.x = reinterpret_cast<const bf16*>(x);
+    a.w = reinterpret_cast<const bf16*>(w);
+    a.bias = reinterpret_cast<const bf16*>(bias);
+    a.M = m;
+    a.N = n;
+    a.K = k;
+    a.y = reinterpret_cast<bf16*>(y);
+    a.ldy = n;
+    return launch_wide_gemm(a, st);
+  }
   if (m <= kSkinnyMaxTok) {
     const bf16* xr[kSkinnyMaxTok];
     bf16* yr[kSkinnyMaxTok];

@@ -98,3 +98,24 @@ print("captured ok")
 """
     p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
     assert p.returncode == 0 and "captured ok" in p.stdout, p.stdout + p.stderr
+
+
+@pytest.mark.parametrize("m,n,k,bias", [
+    (16, 24600, 128, True),    # ragged last tile of 128 columns, two stages
+    (17, 32771, 64, False),    # odd row stride, one stage (fewer than the slots)
+    (32, 32768, 192, False),   # a full 32-row tile
+    (33, 24577, 320, True),    # the 64-row tile, one valid row past 32
+    (64, 28672, 256, False),
+    (1, 500096, 1024, False),  # W of 1 GB: any number of rows
+    (15, 122080, 4096, True),
+])
+def test_wide_decode_products(dev, m, n, k, bias):
+    from swarmlora_amd import ops
+    x, w = randn((m, k), 1).to(dev), torch.empty((n, k), dtype=BF16, device=dev).normal_(0, 0.02)
+    b = randn((n,), 3).to(dev) if bias else None
+    out = torch.full((m + 1, n), 9.0, dtype=BF16, device=dev)
+    ops.gemm(x, w, b, out=out[:m])
+    want = x.float() @ w.float().t() + (b.float() if bias else 0)
+    torch.cuda.synchronize()
+    assert bool((out[m] == 9.0).all())
+    assert_close(out[:m], want, what=f"{m} {n} {k}")
