@@ -1619,8 +1619,20 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
     }
   }
   // DMA instruction q of a stage (W 0 .. WR / 8 - 1, then x): into slot s
+  // The small tiles walk their stages from a start of their own (tile lin
+  // from stage lin % nk, wrapping): rows a power of two apart put the same k
+  // of every row on the same few memory channels, and tiles in lockstep read
+  // little else.  Every tile from stage 0 -> rotated, 32 rows: 28672 x 4096
+  // 51.9 -> 38.5 us (6.1 TB/s), 65536 x 4096 105 -> 84, 128256 x 2048 115 ->
+  // 86, 152064 x 3584 (no power of two) 181 -> 185.  (The large tiles are
+  // bound by MFMA: no gain.)
+  const int rot = SPLIT ? lin % nk : 0;
   auto request_at = [&](int kt, int s, int q) {
     char* st = pg_lds + s * Geo::STAGE;
+    if constexpr (SPLIT) {
+      kt += rot;
+      if (kt >= nk) kt -= nk;
+    }
     constexpr int QW = WR / 8;
     if (q < QW)
       __builtin_amdgcn_global_load_lds((gbl_ptr)(wsrc[q] + (int64_t)kt * PG_K),
@@ -4947,18 +4959,18 @@ int launch_prefill_gemm(TiledArgs a, const PrefillPlan& p, hipStream_t st) {
 // LDS once, K whole, the rows stored straight from the tile.  Bound by the read
 // of W; the K-sliced kernel writes and reads fp32 partials on top of it (28
 // rows of 128256: 29 MB each way, and an epilogue launch).  Two workgroups of
-// two waves a CU, three 20 or 24 KiB stages each.  128256 x 4096 (1.05 GB): 28
-// rows 252 -> 166 us (6.3 TB/s), 64 rows 309 -> 186, one row 198 -> 160.
-// Where the line lies (us, sliced -> this): from 16 rows the partials cost more
-// than the tiles that a last wave leaves idle once there are 3/4 of a tile a CU
-// (16 rows of 28672 x 4096: 53.5 -> 51.2, 36864: 68.6 -> 68.7, 64 rows 71 ->
-// 54; half a tile a CU, 16384 x 4096, 16 rows: 34.5 -> 35.7).  Below 16 rows
-// the partials are small, and only a W of 1 GB makes enough waves of tiles (one
-// row of 152064 x 3584: 216 -> 172; 98304 x 4096: 145 -> 149; 65536 x 4096: 98
-// -> 109).
+// two waves a CU, three 20 or 24 KiB stages each.  us, sliced -> this, for 1 /
+// 28 / 64 rows: 128256 x 4096 198 / 252 / 309 -> 159 / 165 / 184 (6.4 TB/s);
+// 28672 x 8192 97 / 124 / 142 -> 71 / 72 / 76; 28672 x 4096 50 / 61 / 75 -> 38
+// / 39 / 42; 36864 x 4096 (a second workgroup on every eighth CU) 62 / 78 / 94
+// -> 60 / 63 / 71.
+// Where the line lies: 9/16 of a tile a CU for any rows (18944 x 3584, 0.58:
+// 37 / 46 / 60 -> 32 / 33 / 37; 16384 x 4096, 0.50, one row 31.4 -> 33.1), 7/16
+// above 16 rows, where the partials weigh more (14336 x 4096, 0.44, 28 rows
+// 35.4 -> 33.7, 16 rows 31.7 -> 32.9; 11008 x 2048, 0.34, 28 rows 17.7 -> 19.7).
 bool wide_gemm_fits(int64_t m, int64_t n, int64_t k) {
   if (m > kSkinnyMaxTok || k % PG_K != 0 || prefill_uses_tiled(k)) return false;
-  return m >= 16 ? 4 * ((n + 127) / 128) >= 3 * (int64_t)cu_count() : n * k >= 500000000;
+  return 16 * ((n + 127) / 128) >= (m > 16 ? 7 : 9) * (int64_t)cu_count();
 }
 int launch_wide_gemm(TiledArgs a, hipStream_t st) {
   a.n_split = 1;

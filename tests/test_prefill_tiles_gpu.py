@@ -101,13 +101,14 @@ print("captured ok")
 
 
 @pytest.mark.parametrize("m,n,k,bias", [
-    (16, 24600, 128, True),    # ragged last tile of 128 columns, two stages
-    (17, 32771, 64, False),    # odd row stride, one stage (fewer than the slots)
-    (32, 32768, 192, False),   # a full 32-row tile
-    (33, 24577, 320, True),    # the 64-row tile, one valid row past 32
-    (64, 28672, 256, False),
-    (1, 500096, 1024, False),  # W of 1 GB: any number of rows
-    (15, 122080, 4096, True),
+    (16, 18440, 128, True),    # ragged last tile of 128 columns, two stages
+    (17, 14337, 64, False),    # odd row stride, one stage (fewer than the slots)
+    (32, 14336, 192, False),   # a full 32-row tile
+    (33, 14340, 320, True),    # the 64-row tile, one valid row past 32
+    (64, 28672, 256, False),   # tiles starting at each of four stages
+    (1, 18432, 1024, False),
+    (15, 18433, 4096, True),
+    (15, 18304, 64, False),    # one tile short: the K-sliced kernel
 ])
 def test_wide_decode_products(dev, m, n, k, bias):
     from swarmlora_amd import ops
