@@ -5623,27 +5623,30 @@ int swl_lora_delta_bf16(const void* x, int64_t ldx, int64_t m, int64_t k, const 
   r.y = reinterpret_cast<bf16*>(y);
   r.ldy = ldy;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 sgrid((unsigned)((m + kLdRows - 1) / kLdRows), (unsigned)n_ks, (unsigned)((nr + 63) / 64));
-  if (kmajor)
-    hipLaunchKernelGGL(lora_shrink_kernel<true>, sgrid, dim3(512), 0, st, r);
-  else
-    hipLaunchKernelGGL(lora_shrink_kernel<false>, sgrid, dim3(512), 0, st, r);
-  SWL_LAUNCH_CHECK("lora_shrink_kernel launch");
   // rows of an expand workgroup: 64, fewer where that leaves CUs idle (each
   // workgroup reads its columns' B again)
   const int64_t cgroups = (r.tile0[nblk] + 3) / 4;
   const int rt = m <= 16 || cgroups * ((m + 31) / 32) < cu_count() ? 1 : cgroups * ((m + 63) / 64) < cu_count() ? 2 : 4;
   const dim3 egrid((unsigned)cgroups, (unsigned)((m + 16 * rt - 1) / (16 * rt)));
   const int ksn = rank <= 32 ? 1 : 2;
+  // u of the rows and the waves' tiles of B: 65-73 KiB at 64 rows of three
+  // blocks of rank 64 or four of 48 and more (allowed ahead of the shrink)
   const size_t lds = (size_t)16 * rt * (nr + 8) * 2 + (size_t)4 * 8 * ksn * kLdQuad;
-  switch (ksn * 8 + rt) {
-    case 9: hipLaunchKernelGGL((lora_expand_mfma_kernel<1, 1>), egrid, dim3(256), lds, st, r); break;
-    case 10: hipLaunchKernelGGL((lora_expand_mfma_kernel<1, 2>), egrid, dim3(256), lds, st, r); break;
-    case 12: hipLaunchKernelGGL((lora_expand_mfma_kernel<1, 4>), egrid, dim3(256), lds, st, r); break;
-    case 17: hipLaunchKernelGGL((lora_expand_mfma_kernel<2, 1>), egrid, dim3(256), lds, st, r); break;
-    case 18: hipLaunchKernelGGL((lora_expand_mfma_kernel<2, 2>), egrid, dim3(256), lds, st, r); break;
-    default: hipLaunchKernelGGL((lora_expand_mfma_kernel<2, 4>), egrid, dim3(256), lds, st, r); break;
-  }
+  using Expand = void (*)(LoraDeltaArgs);
+  const Expand by_rt[2][3] = {
+      {lora_expand_mfma_kernel<1, 1>, lora_expand_mfma_kernel<1, 2>, lora_expand_mfma_kernel<1, 4>},
+      {lora_expand_mfma_kernel<2, 1>, lora_expand_mfma_kernel<2, 2>, lora_expand_mfma_kernel<2, 4>}};
+  const Expand expand = by_rt[ksn - 1][rt / 2];
+  static size_t allowed = 0;  // (only <2, 4> gets past 64 KiB)
+  int rc = allow_lds(expand, lds, &allowed);
+  if (rc) return rc;
+  const dim3 sgrid((unsigned)((m + kLdRows - 1) / kLdRows), (unsigned)n_ks, (unsigned)((nr + 63) / 64));
+  if (kmajor)
+    hipLaunchKernelGGL(lora_shrink_kernel<true>, sgrid, dim3(512), 0, st, r);
+  else
+    hipLaunchKernelGGL(lora_shrink_kernel<false>, sgrid, dim3(512), 0, st, r);
+  SWL_LAUNCH_CHECK("lora_shrink_kernel launch");
+  hipLaunchKernelGGL(expand, egrid, dim3(256), lds, st, r);
   SWL_LAUNCH_CHECK("lora_expand_mfma_kernel launch");
   return SWL_OK;
 }

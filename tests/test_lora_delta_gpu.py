@@ -28,6 +28,9 @@ def _want(x, fA, bs, rank, alpha):
     (6, 14336, 16, [4096], False, False), (31, 8, 8, [100], False, False), (130, 1000, 64, [333], False, False),
     (48, 544, 56, [37, 91], False, False), (300, 2048, 16, [65, 63, 9, 129], False, False),
     (70, 512, 16, [128, 264], True, False), (70, 512, 48, [128, 264], False, True),
+    # 64-row expand workgroups: more than 64 KiB of LDS from 192 shrink columns on, just below
+    (700, 512, 64, [4096, 1024, 1024], True, True), (641, 264, 48, [2048, 2048, 1032, 1024], True, True),
+    (650, 256, 64, [2048, 2048, 1024, 1024], False, False), (641, 256, 56, [4096, 1024, 1024], True, True),
 ])
 def test_lora_delta_matches_two_products(dev, m, k, rank, cols, kmajor, rr_major):
     from swarmlora_amd import ops
