@@ -2821,7 +2821,7 @@ __device__ __forceinline__ void attn_row(const AttnArgs& a, int s, int h, int gs
     for (int d = 0; d < 8; ++d) stg(dst + d, o[d]);
   }
 }
-  // bytes of a key quad's 128 dims x 4 keys, 128 of skew
+
 // P16: pages are whole 16-key tiles (one cache offset per tile, found 64 tiles
 // at a time); else the offset of every key is looked up.
 template <int KH, bool P16>
@@ -2930,7 +2930,6 @@ __global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, in
   for (int e = 0; e < 2; ++e)
 #pragma unroll
     for (int d = 0; d < 8; ++d) acc[e][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  uint32_t nonfinite = 0;  // V of a step that some rows see part of holds an infinity or NaN
 
   if (nsteps > 0) {
     load_k(0);
@@ -2963,15 +2962,6 @@ __global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, in
         for (int q = 0; q < 4; ++q) {
           const int k = 16 * n + 4 * g + q;
           if (k >= live || (none >> k & 1)) vr[n][q] = u32x4{0u, 0u, 0u, 0u};
-          if (edge) {
-            uint32_t bad = 0;
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-              const uint32_t w = vr[n][q][p];
-              bad |= ((w & 0x7f80u) == 0x7f80u || (w & 0x7f800000u) == 0x7f800000u) ? 1u : 0u;
-            }
-            nonfinite |= bad;
-          }
         }
     }
 #pragma unroll
@@ -3071,15 +3061,26 @@ __global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, in
     __builtin_amdgcn_wave_barrier();  // (LDS accesses of a wave stay in order: the reads precede the next writes)
   }
 
-  if (lane == 0) vbad[kh] = 0;
-  if (__ballot(nonfinite != 0) != 0 && lane == 0) vbad[kh] = 1;
+  // Sums that are not finite, or of 2^100 and more: an infinity or NaN in V is
+  // a NaN in every row of the block (0 times it, in the rows that do not see
+  // its key; in the others the probability's two halves, one of them 0 or
+  // negative, disagree), and the sums run up to 2^8 above their row's
+  // reference, so that V near the largest number overflows early.  These rows
+  // again, key by key in fp32.
+  uint32_t top = 0;
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) top = max(top, __float_as_uint(acc[e][d][q]) & 0x7fffffffu);
+  const bool bad = __ballot(top >= 0x71800000u) != 0;  // 2^100
+  if (lane == 0) vbad[kh] = bad ? 1 : 0;
   __syncthreads();
   uint32_t again = 0;
 #pragma unroll
   for (int w = 0; w < KH; ++w) again |= vbad[w];
   if (again) {  // uniform over the workgroup
-    // such a value's key has probability 0 in a row that does not see it, and
-    // 0 times it is a NaN: these rows again, key by key
     for (int r = r0 + kh; r < min(r0 + 32, rows); r += KH) attn_row(a, s, h, gsh, r, lane);
     return;
   }

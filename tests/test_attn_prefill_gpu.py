@@ -96,22 +96,53 @@ def test_prefill_attention_missing_pages(dev, scale):
 
 
 @pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
-@pytest.mark.parametrize("L,ctx", [(40, 10), (100, 200)])
-def test_prefill_attention_keeps_nonfinite_values_causal(dev, value, L, ctx):
-    """A non-finite value of new token 17 reaches the rows that see it and no
-    other; non-finite cache contents past the context reach none."""
+@pytest.mark.parametrize("L,ctx,at", [(40, 10, 27), (100, 200, 217), (100, 200, 3), (70, 300, 299), (33, 1000, 500)])
+def test_prefill_attention_keeps_nonfinite_values_causal(dev, value, L, ctx, at):
+    """A non-finite value of key `at` (a new token, or one of the cached context,
+    which every row sees) gives the rows that see it what the definition gives
+    (inf, -inf or NaN) and reaches no other; with an infinity of the other sign
+    beside it, NaN.  Non-finite cache contents past the context reach none."""
     c = _case(dev, 1, L, 8, 2, [ctx], 16)
     clean, _ = _run(dev, {k: v.clone() for k, v in c.items()}, 128 ** -0.5)
-    c["v"][0, 17, 1, 5] = value
+
+    def put(key, x, dim):
+        if key < ctx:
+            c["vc"][int(c["bt"][0, key // 16]), key % 16, 1, dim] = x
+        else:
+            c["v"][0, key - ctx, 1, dim] = x
+    put(at, value, 5)
+    put(at, value, 77)
+    put(min(at + 2, ctx + L - 1), -value, 77)
     c["vc"][int(c["bt"][0, -1])] = math.nan   # a page past every context
     c["kc"][int(c["bt"][0, -1])] = math.nan
     got, _ = _run(dev, c, 128 ** -0.5)
+    seen = torch.arange(L) + ctx >= at
+    both = torch.arange(L) + ctx >= at + 2
+    got, clean = got.view(L, 8, 128), clean.view(L, 8, 128)
     hit = torch.zeros(L, 8, 128, dtype=torch.bool)
-    hit[17:, 4:, 5] = True  # kv head 1 serves query heads 4..7
-    hit = hit.reshape(1, L, -1)
-    assert not bool(got[hit].isfinite().any())
+    hit[:, 4:, 5], hit[:, 4:, 77] = seen[:, None], seen[:, None]  # kv head 1 serves query heads 4..7
+    want = torch.full_like(got, value)
+    want[both, :, 77] = math.nan
+    assert bool(((got == want) | (got.isnan() & want.isnan()))[hit].all())
     # the rest as without it; rows computed key by key round differently
     assert float((got[~hit] - clean[~hit]).abs().max()) <= 4e-3 * 6.0
+
+
+@pytest.mark.parametrize("at", [280, 301])
+def test_prefill_attention_values_near_the_largest_number(dev, at):
+    """V of 3e38 at a key whose score is 5 above the others', which come first:
+    the weighted sum stays finite (the weights are at most 1)."""
+    L, ctx, big = 20, 300, 3e38
+    c = _case(dev, 1, L, 8, 2, [ctx], 16)
+    c["q"].fill_(1.0)
+    c["k"].zero_(), c["kc"].zero_()
+    if at < ctx:
+        c["kc"][int(c["bt"][0, at // 16]), at % 16] = 1.0
+        c["vc"][int(c["bt"][0, at // 16]), at % 16] = big
+    else:
+        c["k"][0, at - ctx], c["v"][0, at - ctx] = 1.0, big
+    got, _ = _run(dev, c, 5.0 / 128)
+    _check(got, _want(c, 5.0 / 128), big)
 
 
 def test_prefill_attention_under_capture_without_a_first_call(dev):
