@@ -6412,10 +6412,13 @@ int round_launch_ws(int n_seg, const int64_t* rows, const void* const* seg_in, v
     a.L.usplit = 1;  // folded into split 0
     a.L.u_ld = u_ld;
     a.L.u_split_stride = (int64_t)T * u_ld;
-    // the 256 x 256 kernel adds the LoRA delta as MFMA k-steps when every
-    // tile lies inside one column block and the ranks are multiples of 8
+    // The LoRA delta as MFMA k-steps of the tiles, u * scale rounded to bf16,
+    // when every 256-column tile lies inside one column block and the ranks
+    // are multiples of 8.  Any other round adds it in fp32 in the epilogue,
+    // also where 128-column tiles would lie inside the blocks: how a round is
+    // tiled does not decide the delta's precision.
     a.lora_mfma = 1;
-    for (int b = 1; b < nblk; ++b) a.lora_mfma &= (L.blk_start[b] % (plan.rows == 0 ? 128 : PG_N) == 0) ? 1 : 0;
+    for (int b = 1; b < nblk; ++b) a.lora_mfma &= (L.blk_start[b] % PG_N == 0) ? 1 : 0;
     for (int i = 0; i < n_seg; ++i)
       if (a.seg_lora[i] >= 0) {
         const int r = host_entries[a.seg_lora[i]].rank;

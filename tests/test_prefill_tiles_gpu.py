@@ -58,6 +58,30 @@ def test_short_prefill_rounds(dev, rows, n, k, cols, ranks, bias):
         assert_close(g, w, what=f"{rows} {n} {k}")
 
 
+@pytest.mark.parametrize("rows,k,cols", [([70], 512, [128, 256]), ([90, 60], 4096, [384, 640, 256])])
+def test_short_prefill_delta_off_the_large_grid_in_fp32(dev, rows, k, cols):
+    """Column blocks at multiples of 128 that are none of 256: the delta is
+    fp32 up to the result's one rounding (half a bf16 step is at most 2^-8 of
+    the value; 1e-5 of the largest for the fp32 sums over k)."""
+    from swarmlora_amd import ops
+    n, r = sum(cols), 8
+    w = torch.zeros(n, k, dtype=BF16, device=dev)
+    table, ids, xs, want = ops.LoraTable(dev), [], [], []
+    for i, m in enumerate(rows):
+        x, a = randn((m, k), i), randn((r * len(cols), k), 10 + i, std=0.05)
+        bs = [randn((c, r), 20 + 5 * i + j) for j, c in enumerate(cols)]
+        u = 1.7 * (x.double() @ a.double().t())
+        want.append(torch.cat([u[:, j * r:(j + 1) * r] @ b.double().t() for j, b in enumerate(bs)], 1))
+        ids.append(table.add(a.to(dev), [b.to(dev) for b in bs], r, 1.7))
+        xs.append(x.to(dev))
+    outs = [torch.zeros(m, n, dtype=BF16, device=dev) for m in rows]
+    ops.round_fused(xs, outs, rows, w, None, seg_lora=ids, table=table, blk_cols=cols)
+    torch.cuda.synchronize()
+    for o, y in zip(outs, want):
+        err = (o.double().cpu() - y).abs() - 2 ** -8 * y.abs()
+        assert float(err.max()) <= 1e-5 * float(y.abs().max())
+
+
 def test_short_prefill_round_captured_without_room_for_splits(dev):
     """A captured round that would need more scratch for its splits than the
     library holds runs unsplit (its shrink fits what an earlier call sized),
