@@ -1326,7 +1326,7 @@ struct TiledArgs {
   int32_t n_split;
   float* part;
   // first row of the 128 x 128 tiles: the rows before it have large tiles in
-  // a launch of their own (whose M ends there)
+  // a launch of their own (whose M ends there; no K split then)
   int64_t m_base;
 };
 
@@ -1618,15 +1618,17 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
       xsrc[i] = a.xin[sg] + (mr - a.out.off[sg]) * a.K + (int64_t)kt0 * PG_K + 8 * dc;
     }
   }
-  // DMA instruction q of a stage (W 0 .. WR / 8 - 1, then x): into slot s
-  // The small tiles walk their stages from a start of their own (tile lin
-  // from stage lin % nk, wrapping): rows a power of two apart put the same k
+  // The small tiles walk their stages from a start of their own (column tile
+  // c from stage c % nk, wrapping): rows a power of two apart put the same k
   // of every row on the same few memory channels, and tiles in lockstep read
   // little else.  Every tile from stage 0 -> rotated, 32 rows: 28672 x 4096
   // 51.9 -> 38.5 us (6.1 TB/s), 65536 x 4096 105 -> 84, 128256 x 2048 115 ->
   // 86, 152064 x 3584 (no power of two) 181 -> 185.  (The large tiles are
-  // bound by MFMA: no gain.)
-  const int rot = SPLIT ? lin % nk : 0;
+  // bound by MFMA: no gain.)  The start depends on the column alone, and
+  // tiles behind large ones walk as those do: every row of a round adds its
+  // products in the same order, wherever in the batch it is.
+  const int rot = SPLIT && a.m_base == 0 ? (int)(n0 / NT) % nk : 0;
+  // DMA instruction q of a stage (W 0 .. WR / 8 - 1, then x): into slot s
   auto request_at = [&](int kt, int s, int q) {
     char* st = pg_lds + s * Geo::STAGE;
     if constexpr (SPLIT) {
@@ -1688,6 +1690,9 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
       my.b = *(const __attribute__((address_space(1))) bptr*)(ep + offsetof(swl_lora_entry, b) + lb * sizeof(void*));
       my.rank = *(const __attribute__((address_space(1))) int32_t*)(ep + offsetof(swl_lora_entry, rank));
       my.scale = *(const __attribute__((address_space(1))) float*)(ep + offsetof(swl_lora_entry, scale));
+      // K split: each adapter's steps in one split, by its table index (not by
+      // the segment's place in the tile: see rot)
+      if (SPLIT && e % a.n_split != sp) my.rank = 0;
     }
   }
 #pragma unroll
@@ -1776,12 +1781,11 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
   // bf16 (zero for the other segments' rows), 16 ranks a step.  The steps
   // run as one loop over (segment, rank step) with the next step's loads in
   // flight while the current one's MFMAs issue (two register sets taking
-  // turns), the entries read from the tile's LDS table.  With K split, the
-  // segments are dealt over the splits.
+  // turns), the entries read from the tile's LDS table.
   if (lora_k) {
     const int64_t bstart = blk_start_of(a.L, lb);
-    auto first = [&](int i) {  // first segment from i with an adapter (of this split's)
-      while (i < nseg && (segl[i].rank <= 0 || (SPLIT && i % a.n_split != sp))) ++i;
+    auto first = [&](int i) {  // first segment from i with an adapter
+      while (i < nseg && segl[i].rank <= 0) ++i;
       return i;
     };
     auto advance = [&](int& i, int& q0) {
@@ -1914,7 +1918,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
           const int tr = (threadIdx.x >> 4) + RG * kk;
           const f32x4 q = *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(pg_lds) + (w2 * TPW + tr) * ELD + 4 * cq);
           const int64_t m = m0 + (w2 >> 1) * TPW + tr, n = n0 + (w2 & 1) * CPW + 64 * h + 4 * cq;
-          float* dst = a.part + ((int64_t)sp * (a.M - a.m_base) + m - a.m_base) * a.N + n;
+          float* dst = a.part + ((int64_t)sp * a.M + m) * a.N + n;
           if (m >= a.M || n >= a.N) continue;
           if ((a.N & 3) == 0) {
             *(__attribute__((address_space(1))) f32x4*)(dst) = q;
@@ -1959,14 +1963,14 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm256_kernel(TiledArgs a, int t
 // bias (and the LoRA delta where the tiles could not carry it), one rounding,
 // the row's slot.  One thread per 4 columns of a row.
 __global__ __launch_bounds__(256) void prefill_fold_kernel(TiledArgs a) {
-  const int64_t m = a.m_base + blockIdx.y;
+  const int64_t m = blockIdx.y;
   const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (n >= a.N) return;
   const int sg = a.y ? 0 : find_seg(a.out.off, a.out.n, m);
   bf16* yrow = a.y ? a.y + m * a.ldy
                    : reinterpret_cast<bf16*>(const_cast<void*>(a.out.ptr[sg])) + (m - a.out.off[sg]) * a.N;
-  const float* p = a.part + (int64_t)blockIdx.y * a.N + n;
-  const int64_t stride = (a.M - a.m_base) * a.N;
+  const float* p = a.part + m * a.N + n;
+  const int64_t stride = a.M * a.N;
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   for (int k0 = 0; k0 < a.n_split; k0 += 4) {
     f32x4 q[4];
@@ -4925,7 +4929,7 @@ PrefillPlan plan_prefill(int64_t M, int64_t N, int64_t K, bool split_ok) {
     for (int64_t rows = 64 * nj; rows < M; rows += 64 * nj) {
       const double t = large(nj, rows, (double)((rows / (64 * nj) * tiles_n + cus - 1) / cus) * (nj == 3 ? 0.9 : 1.0)) + 8.0;
       if (t >= best) break;
-      for (int s = 1; s <= most; ++s) take(t + small(M - rows, s), nj, rows, s);
+      take(t + small(M - rows, 1), nj, rows, 1);
     }
   return p;
 }
@@ -4946,11 +4950,11 @@ int launch_prefill_gemm(TiledArgs a, const PrefillPlan& p, hipStream_t st) {
     if (rc || p.rows >= a.M) return rc;
   }
   a.m_base = p.rows;
-  if (a.part) a.n_split = p.n_split;
+  if (a.part && p.rows == 0) a.n_split = p.n_split;
   int rc = a.M - a.m_base <= 128 ? launch_gemm256<2, 2, 2, 4, true>(a, st) : launch_gemm256<2, 2, 2, 4>(a, st);
   if (rc || !a.part) return rc;
-  hipLaunchKernelGGL(prefill_fold_kernel, dim3((unsigned)((a.N + 1023) / 1024), (unsigned)(a.M - a.m_base)),
-                     dim3(256), 0, st, a);
+  hipLaunchKernelGGL(prefill_fold_kernel, dim3((unsigned)((a.N + 1023) / 1024), (unsigned)a.M), dim3(256), 0, st,
+                     a);
   SWL_LAUNCH_CHECK("prefill_fold_kernel launch");
   return SWL_OK;
 }
@@ -6368,7 +6372,7 @@ int round_launch_ws(int n_seg, const int64_t* rows, const void* const* seg_in, v
   // of it than there is
   const size_t ubytes_al = (ubytes + 255) & ~(size_t)255;
   PrefillPlan plan = plan_prefill(T, N, K, has_lora && !packed_x && T <= 65535);
-  size_t pbytes = plan.n_split > 1 ? sizeof(float) * (size_t)plan.n_split * (size_t)(T - plan.rows) * (size_t)N : 0;
+  size_t pbytes = plan.n_split > 1 ? sizeof(float) * (size_t)plan.n_split * (size_t)T * (size_t)N : 0;
   if (pbytes && !scratch_may_hold(xbytes_al + ubytes_al + pbytes, st)) {
     plan.n_split = 1;
     pbytes = 0;

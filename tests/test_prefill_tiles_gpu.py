@@ -124,6 +124,36 @@ print("captured ok")
     assert p.returncode == 0 and "captured ok" in p.stdout, p.stdout + p.stderr
 
 
+@pytest.mark.parametrize("rows,n,k,cols,same", [
+    ([150, 300, 150], 2048, 4096, [1024, 1024], (0, 2)),       # 128 x 128 tiles, K split
+    ([200] + [1] * 40, 4096, 8192, [4096], (1, 20, 40)),       # one-row slots of two row tiles
+    ([130, 1, 200, 130], 2304, 4096, None, (0, 3)),            # no adapters: unsplit
+    ([90, 40, 90], 456, 4096, [200, 256], (0, 2)),             # the delta in the splits' sum
+    ([300] * 9, 6144, 4096, [4096, 1024, 1024], (0, 4, 8)),    # large tiles, then 128 x 128
+    ([300] * 9, 6144, 4096, None, (0, 8)),
+    ([700, 700, 700], 2048, 1024, [2048], (0, 1, 2)),
+])
+def test_a_prompt_gives_the_same_bits_wherever_it_is_in_the_round(dev, rows, n, k, cols, same):
+    """Segments of the same rows and adapter: every row adds its products in
+    the same order, in whichever tile, launch or split it lands."""
+    from swarmlora_amd import ops
+    w, b = randn((n, k), 0, std=0.02).to(dev), randn((n,), 1).to(dev)
+    table, nb = ops.LoraTable(dev), len(cols or [])
+    xs, ids = [], []
+    for i, r in enumerate(rows):
+        j = same[0] if i in same else i
+        xs.append(xs[j].clone() if i in same[1:] else randn((r, k), 2 + i).to(dev))
+        if cols:
+            ids.append(ids[j] if i in same[1:] else table.add(
+                randn((16 * nb, k), 100 + i, std=0.02).to(dev), [randn((c, 16), 200 + i, std=0.02).to(dev) for c in cols],
+                16, 2.0))
+    outs = [torch.zeros(r, n, dtype=BF16, device=dev) for r in rows]
+    ops.round_fused(xs, outs, rows, w, b, seg_lora=ids or None, table=table if cols else None, blk_cols=cols)
+    torch.cuda.synchronize()
+    for i in same[1:]:
+        assert torch.equal(outs[i], outs[same[0]]), f"segment {i}"
+
+
 @pytest.mark.parametrize("m,n,k,bias", [
     (16, 18440, 128, True),    # ragged last tile of 128 columns, two stages
     (17, 14337, 64, False),    # odd row stride, one stage (fewer than the slots)
