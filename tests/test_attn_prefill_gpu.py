@@ -145,6 +145,22 @@ def test_prefill_attention_values_near_the_largest_number(dev, at):
     _check(got, _want(c, 5.0 / 128), big)
 
 
+def test_prefill_attention_nan_scores_cost_no_recomputation(dev):
+    """A NaN in q, or in a key, makes 0 of the rows it reaches; the others keep
+    their bits (the block is not computed again key by key)."""
+    c = _case(dev, 1, 50, 8, 2, [300], 16)
+    clean, _ = _run(dev, {k: v.clone() for k, v in c.items()}, 128 ** -0.5)
+    clean = clean.view(50, 8, 128)
+    c["q"][0, 7, 2] = math.nan
+    c["k"][0, 20, 1] = math.nan    # kv head 1: query heads 4..7 of tokens 20..
+    got, _ = _run(dev, c, 128 ** -0.5)
+    got = got.view(50, 8, 128)
+    hit = torch.zeros(50, 8, dtype=torch.bool)
+    hit[7, 2], hit[20:, 4:] = True, True
+    assert bool((got[hit] == 0).all())
+    assert torch.equal(got[~hit], clean[~hit])
+
+
 def test_prefill_attention_under_capture_without_a_first_call(dev):
     """The kernel takes no scratch: a graph can capture the first call ever
     made with a shape, and replays give the eager result each time."""
