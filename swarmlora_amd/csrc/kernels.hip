@@ -4862,16 +4862,10 @@ int launch_gemm256(const TiledArgs& a, hipStream_t st, hipEvent_t e0 = nullptr, 
 
 // Tile of a prefill GEMM (nj: 4 = 256 x 256, 3 = 256 x 192, 2 = 128 x 128) and
 // the K splits of the last, by estimated time; `split_ok`: the caller has
-// scratch for the splits' fp32 tiles.  The 128 x 128 tile runs at 0.7 of the
-// large ones' rate once they fill the chip, but a short batch leaves most CUs
-// without a large tile: measured per round with rank-16 adapters, large ->
-// 128 x 128 (us), 107 rows: QKV 104 -> 34, O 102 -> 31, Gate+Up 87 -> 54, Down
-// 305 -> 53; 512 rows: 97 -> 55, 94 -> 44, 134 -> 176 (kept large), 281 -> 97;
-// 1000 rows: 98 -> 96, 94 -> 55, 259 -> 323 (large), 274 -> 154; level or
-// large from ~1500 rows.
-// Rows that would start another wave of large tiles go to 128 x 128 tiles
-// behind them: 2997 rows, QKV: 16 x 24 tiles of 192 rows, 1.5 waves; 10 x 24
-// of 256 rows, then 437 rows in 128 x 128 tiles (201 -> 164 us).
+// scratch for the splits' fp32 tiles.  The large tiles do the most per byte,
+// but a short batch leaves most CUs without one, and a batch just past a
+// whole number of waves starts another for a few rows: those rows then go to
+// 128 x 128 tiles in a launch behind.
 struct PrefillPlan {
   int nj = 4;           // of the rows before `rows`
   int64_t rows = 0;     // in large tiles; the rest in 128 x 128 tiles
@@ -4884,42 +4878,45 @@ PrefillPlan plan_prefill(int64_t M, int64_t N, int64_t K, bool split_ok) {
     return e ? atoi(e) : 0;
   }();
   const int64_t cus = cu_count(), stages = K / PG_K;
-  // Large tiles, in tile times: 256 token rows, or 192 where the grid then
-  // covers the CUs in fewer of them (a 192-row tile measured at ~0.9 of a
-  // 256-row one: the W side streams the same bytes): the O and Down rounds at
-  // 2325 rows have 160 tiles of 256 for 256 CUs, 208 of 192 (146 -> 133 us,
-  // 370 -> 335).  A tile of the last row tile costs the share of its first row
-  // wave's 32-row blocks that hold rows, at least 0.4 of a full tile (its
-  // stages still wait for their DMA); such tiles first fill the CUs the last
-  // wave of full tiles leaves idle, and where they do not fit there they
-  // start another.
   const int64_t tiles_n = (N + PG_N - 1) / PG_N;
-  auto cost = [&](int nj) {
-    const int64_t mt = 64 * nj, full = (M / mt) * tiles_n, rem = M % mt;
+  // The estimates (us) are fitted to 380 shapes, with a rank-16 adapter and
+  // without, 65 to 4096 rows of ten weights (2048 x 2048 to 28672 x 4096 and
+  // 3584 x 18944) read from memory: every tiling and split of each was timed.
+  // What the rule takes is 0.2 % behind the best on average and at most 4 %
+  // behind large tiles alone.  Large tiles alone -> taken, with an adapter: 128
+  // rows, 6144 x 4096 98 -> 35, 4096 x 4096 97 -> 31, 28672 x 4096 108 -> 60,
+  // 4096 x 14336 303 -> 48; 512 rows 92 -> 52, 92 -> 42, 122 (large), 279 ->
+  // 95; 1000 rows 92 -> 91, 89 -> 52, 228 (large), 268 -> 155; 2997 rows 195 ->
+  // 159 (2560 rows in large tiles), the others large.
+  //
+  // Large tiles, in waves of one a CU: 1.1 a stage (1.02 with 192 rows) and
+  // 0.16 (0.13) more with every CU busy (the clock falls with the load), 12.5
+  // for the ramp and the epilogue, and the reads of W, which only the first
+  // row tile takes from memory.  A tile of the last row tile costs the share
+  // of its first row wave's 32-row blocks that hold rows, at least 0.4 (its
+  // stages still wait for their DMA); such tiles first fill the CUs that the
+  // last wave of full tiles leaves idle, and where they do not fit there they
+  // start another.
+  auto large = [&](int nj, int64_t rows) {
+    const int64_t mt = 64 * nj, full = rows / mt * tiles_n, rem = rows % mt;
     const double pc = rem ? std::max(0.4, (double)std::min<int64_t>(nj, (rem + 31) / 32) / nj) : 0.0;
     const int64_t waves = (full + cus - 1) / cus;
     const int64_t spill = (rem ? tiles_n : 0) - (waves * cus - full);
-    const double t = (double)waves + (spill > 0 ? (double)((spill + cus - 1) / cus) * pc : 0.0);
-    return t * (nj == 3 ? 0.9 : 1.0);
+    const int64_t more = spill > 0 ? (spill + cus - 1) / cus : 0;
+    const double busy = ((double)full + pc * (double)tiles_n) / (double)cus;
+    return (double)stages * (((double)waves + (double)more * pc) * (nj == 3 ? 1.02 : 1.1) + busy * (nj == 3 ? 0.13 : 0.16)) +
+           (double)(waves + more) * (12.5 + (double)stages / (double)((rows + mt - 1) / mt));
   };
-  p.nj = forced == 3 || forced == 4 ? forced : cost(3) < cost(4) ? 3 : 4;
-  p.rows = M;
-  if (forced == 3 || forced == 4) return p;
-  // us: a large tile's stage takes 1.25 with few CUs busy, 1.85 with all (the
-  // clock falls with the load); a 128 x 128 stage 0.65, the splits' sum a
-  // launch (5) and their bytes, written and read, at 4 TB/s; a second launch 8
-  // (the first one's last tiles, and its own ramp)
-  auto large = [&](int nj, int64_t rows, double waves) {
-    const int64_t tiles = (rows + 64 * nj - 1) / (64 * nj) * tiles_n;
-    return waves * (double)stages * (1.25 + 0.6 * std::min(1.0, (double)tiles / (double)cus));
-  };
+  // 128 x 128 tiles: a stage slows with the tiles in flight (they pull their
+  // operands through the same L2s); the splits' sum costs a launch and their
+  // fp32 tiles, written and read at 4.9 TB/s.
   auto small = [&](int64_t rows, int s) {
-    const int64_t tiles = (rows + 127) / 128 * ((N + 127) / 128);
-    return (double)((tiles * s + cus - 1) / cus) * (double)((stages + s - 1) / s) * 0.65 +
-           (s > 1 ? 5.0 + (double)(s * rows * N) * 8.0 / 4e6 : 0.0);
+    // (every XCD takes an eighth of the tiles, rounded up, in each split)
+    const int64_t tiles = ((rows + 127) / 128 * ((N + 127) / 128) + 7) / 8 * 8 * s, waves = (tiles + cus - 1) / cus;
+    return (double)((stages + s - 1) / s) * (0.41 * (double)waves + 0.21 * (double)tiles / (double)cus) +
+           6.5 * (double)waves + (s > 1 ? 1.0 + (double)(s * rows * N) * 8.0 / 4.9e6 : 0.0);
   };
-  const int most = split_ok ? (int)std::max<int64_t>(1, std::min<int64_t>(16, stages / 4)) : 1;
-  double best = forced == 2 ? 1e30 : large(p.nj, M, cost(p.nj));
+  double best = 1e30;
   auto take = [&](double t, int nj, int64_t rows, int s) {
     if (t < best) {
       best = t;
@@ -4928,14 +4925,14 @@ PrefillPlan plan_prefill(int64_t M, int64_t N, int64_t K, bool split_ok) {
       p.n_split = s;
     }
   };
+  for (int nj = 3; nj <= 4; ++nj)
+    if (forced != 2 && forced != 7 - nj) take(large(nj, M), nj, M, 1);
+  if (forced == 3 || forced == 4) return p;
+  const int most = split_ok ? (int)std::max<int64_t>(1, std::min<int64_t>(16, stages / 4)) : 1;
   for (int s = 1; s <= most; ++s) take(small(M, s), 4, 0, s);
   if (forced == 2) return p;
   for (int nj = 3; nj <= 4; ++nj)
-    for (int64_t rows = 64 * nj; rows < M; rows += 64 * nj) {
-      const double t = large(nj, rows, (double)((rows / (64 * nj) * tiles_n + cus - 1) / cus) * (nj == 3 ? 0.9 : 1.0)) + 8.0;
-      if (t >= best) break;
-      take(t + small(M - rows, 1), nj, rows, 1);
-    }
+    for (int64_t rows = 64 * nj; rows < M; rows += 64 * nj) take(large(nj, rows) + small(M - rows, 1) + 2.0, nj, rows, 1);
   return p;
 }
 
