@@ -4235,39 +4235,35 @@ std::mutex g_scratch_mu;
 std::vector<Scratch> g_scratch;
 std::vector<void*> g_scratch_kept;
 
-int scratch_get(size_t need, hipStream_t stream, void** out) {
+// `optional`: the caller does without where there is no room; *out is null
+// then, with no error left behind.
+int scratch_get(size_t need, hipStream_t stream, void** out, bool optional = false) {
   int dev = 0;
   SWL_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   if ((int)g_scratch.size() <= dev) g_scratch.resize(dev + 1);
   Scratch& s = g_scratch[dev];
   if (s.bytes < need) {
+    *out = nullptr;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (stream) SWL_HIP(hipStreamIsCapturing(stream, &cs));
+    if (optional && cs != hipStreamCaptureStatusNone) return SWL_OK;
     SWL_CHECK(cs == hipStreamCaptureStatusNone, SWL_ERR_STATE,
               "scratch must grow outside graph capture (run the call once before capturing)");
     size_t nb = std::max({need, s.bytes + s.bytes / 2, (size_t)1 << 20});
     nb = (nb + 4095) & ~(size_t)4095;
     void* p = nullptr;
-    SWL_HIP(hipMalloc(&p, nb));
+    if (optional && hipMalloc(&p, nb) != hipSuccess) {
+      (void)hipGetLastError();
+      return SWL_OK;
+    }
+    if (!p) SWL_HIP(hipMalloc(&p, nb));
     if (s.ptr) g_scratch_kept.push_back(s.ptr);
     s.ptr = p;
     s.bytes = nb;
   }
   *out = s.ptr;
   return SWL_OK;
-}
-
-// Whether scratch_get would give `need` bytes: it has them, or may grow.
-bool scratch_may_hold(size_t need, hipStream_t stream) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  {
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (dev < (int)g_scratch.size() && g_scratch[dev].bytes >= need) return true;
-  }
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  return !stream || (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone);
 }
 
 // ---------------------------------------------------------- launch timer
@@ -6370,18 +6366,22 @@ int round_launch_ws(int n_seg, const int64_t* rows, const void* const* seg_in, v
   if (has_lora) ubytes = sizeof(float) * (size_t)u_ks * (size_t)T * (size_t)u_ld;
   // K splits only where the round takes scratch anyway (its LoRA shrink): a
   // round without adapters stays free of it, so such rounds on several
-  // streams stay independent; and not where a captured round would need more
-  // of it than there is
+  // streams stay independent.  Where the scratch has no room for the splits'
+  // tiles, and may not grow (under capture) or cannot, the round is planned
+  // again without them: what ran without splits still runs.  (A round captured
+  // after the same round ran once finds the room and takes the same plan.)
   const size_t ubytes_al = (ubytes + 255) & ~(size_t)255;
   PrefillPlan plan = plan_prefill(T, N, K, has_lora && !packed_x && T <= 65535);
   size_t pbytes = plan.n_split > 1 ? sizeof(float) * (size_t)plan.n_split * (size_t)T * (size_t)N : 0;
-  if (pbytes && !scratch_may_hold(xbytes_al + ubytes_al + pbytes, st)) {
-    plan.n_split = 1;
-    pbytes = 0;
-  }
   void* scr = nullptr;
-  int rc = scratch_get(xbytes_al + (pbytes ? ubytes_al + pbytes : ubytes), st, &scr);
+  int rc = pbytes ? scratch_get(xbytes_al + ubytes_al + pbytes, st, &scr, true) : SWL_OK;
   if (rc) return rc;
+  if (!scr) {
+    if (pbytes) plan = plan_prefill(T, N, K, false);
+    pbytes = 0;
+    rc = scratch_get(xbytes_al + ubytes, st, &scr);
+    if (rc) return rc;
+  }
   bf16* packed = reinterpret_cast<bf16*>(scr);
   if (packed_x) {
     rc = swl_gather_bf16(seg_in, rows, n_seg, K, packed, st);
