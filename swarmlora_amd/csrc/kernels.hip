@@ -3882,7 +3882,8 @@ __device__ __forceinline__ T block_suffix(T v, T* sh) {
 // found in an order-preserving 16-bit key by two histogram levels (4096 bins
 // of 16 keys, then the 16 keys of the bin the threshold falls in) instead of
 // a binary search that reads the row once per step: 2 to 4 passes over the
-// row where there were up to 64.  Probability masses are summed as integers
+// row where there were up to 64.  Without thresholds the histogram is left
+// out: 28 rows of 128256 206 -> 36 us, one of 1000, all latency, 7.2 -> 7.8.  Probability masses are summed as integers
 // (2^44 per unit, less for vocabularies over 2^18, so that no sum passes
 // 2^62): the same sum in any order, at an absolute step of 6e-14.  What
 // bounds it is one CU's vector and LDS-atomic work on a row; 28 rows of
@@ -3968,30 +3969,28 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
   const float P = a.top_p[row];
   const bool by_k = K > 0 && K < V, by_p = P < 1.0f;
 
-  // level 1: mass and count of every bin (only the NaN check when neither
-  // threshold is asked for)
-  for (int i = tid; i < kSampleBins; i += 1024) {
-    mass_bin[i] = 0;
-    cnt_bin[i] = 0;
-  }
   if (tid == 0) nan_key = 0;
-  __syncthreads();
-  for_row([&](uint32_t b, int64_t i) {
-    const float e = prob(b);
-    const uint32_t k = key16(b);
-    if (e != e) {
-      if (i < V) atomicMax(&nan_key, k + 1);
-    } else if (by_k || by_p) {
-      const u64 m = mass_of(e);
-      if (m) atomicAdd(&mass_bin[k >> 4], m);
-    }
-    if (by_k) atomicAdd(&cnt_bin[k >> 4], 1u);
-  });
-  __syncthreads();
-  // masses and counts above each thread's 4 bins
+  // level 1: mass and count of every bin, and of those above each thread's 4
   u64 m4[4], m_own = 0, m_above = 0;
   uint32_t c4[4], c_own = 0, c_above = 0;
   if (by_k || by_p) {
+    for (int i = tid; i < kSampleBins; i += 1024) {
+      mass_bin[i] = 0;
+      cnt_bin[i] = 0;
+    }
+    __syncthreads();
+    for_row([&](uint32_t b, int64_t i) {
+      const float e = prob(b);
+      const uint32_t k = key16(b);
+      if (e != e) {
+        if (i < V) atomicMax(&nan_key, k + 1);
+      } else {
+        const u64 m = mass_of(e);
+        if (m) atomicAdd(&mass_bin[k >> 4], m);
+      }
+      if (by_k) atomicAdd(&cnt_bin[k >> 4], 1u);
+    });
+    __syncthreads();
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       m4[q] = mass_bin[4 * tid + q];
@@ -4074,7 +4073,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
   } else if (by_p) {
     z = block_reduce<u64>(m_own, add64, sh64);
   }
-  if (nan_key > tk) {  // a NaN in the kept set: the most likely token
+  if ((by_k || by_p) && nan_key > tk) {  // a NaN in the kept set: the most likely token
     if (tid == 0) a.out_tok[row][0] = amax;
     return;
   }
@@ -4131,62 +4130,111 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
   };
   // (logits past the row are NaN: fmaxf makes their mass 0)
   __syncthreads();
-  for (int g0 = wv; g0 < ngrp; g0 += 4 * 16) {
-    u64 sum[4] = {0, 0, 0, 0};
-    for (int64_t c = 0; c < per; ++c) {
-      u32x4 q[4];
+  // FIRST: no threshold was asked for, so this is the first look at the
+  // probabilities, and at their NaN
+  auto group_masses = [&](auto first) {
+    constexpr bool FIRST = decltype(first)::value;
+    bool nan = false;
+    for (int g0 = wv; g0 < ngrp; g0 += 4 * 16) {
+      u64 sum[4] = {0, 0, 0, 0};
+      for (int64_t c = 0; c < per; ++c) {
+        u32x4 q[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = block_piece(g0 + 16 * u < ngrp ? (int64_t)(g0 + 16 * u) * per + c : nblk);
+        for (int u = 0; u < 4; ++u) q[u] = block_piece(g0 + 16 * u < ngrp ? (int64_t)(g0 + 16 * u) * per + c : nblk);
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < 4; ++u) {
+          if (FIRST && g0 + 16 * u >= ngrp) break;
+          const int64_t left = V - (((int64_t)(g0 + 16 * u) * per + c) * 512 + 8 * lane);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum[u] += kept_mass(q[u], e);
+          for (int e = 0; e < 8; ++e) {
+            if constexpr (FIRST) {
+              const float p = prob(bits_of(q[u], e));
+              nan |= p != p && e < left;
+              sum[u] += mass_of(fmaxf(p, 0.f));
+            } else {
+              sum[u] += kept_mass(q[u], e);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) sum[u] += __shfl_xor(sum[u], o, 64);
+        if (lane == 0 && g0 + 16 * u < ngrp) mass_bin[g0 + 16 * u] = sum[u];
+      }
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) sum[u] += __shfl_xor(sum[u], o, 64);
-      if (lane == 0 && g0 + 16 * u < ngrp) mass_bin[g0 + 16 * u] = sum[u];
-    }
-  }
+    if (FIRST && __ballot(nan) != 0 && lane == 0) nan_key = 1;
+  };
+  if (by_k || by_p)
+    group_masses(std::false_type{});
+  else
+    group_masses(std::true_type{});
   __syncthreads();
-  // groups 4 tid .. + 3 of this thread; prefix = all - suffix
-  u64 own = 0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    m4[q] = 4 * tid + q < ngrp ? mass_bin[4 * tid + q] : 0;
-    own += m4[q];
+  if (!by_k && !by_p && nan_key) {
+    if (tid == 0) a.out_tok[row][0] = amax;
+    return;
   }
-  const u64 suffix = block_suffix<u64>(own, sh64);
-  __syncthreads();
-  if (tid == 0) {
-    found_above = suffix;  // the whole mass
-    found_bin = -1;
-  }
-  __syncthreads();
-  u64 before = found_above - suffix;
+  // the group that the target falls in, and the mass before it
   const uint64_t r = mix64(a.seed * 0x9e3779b97f4a7c15ull + (uint64_t)row + 1);
-  const u64 target = __umul64hi(found_above, (r >> 40) << 40);  // floor(mass * r24 / 2^24)
-  __syncthreads();
+  auto target_of = [&](u64 all) { return (u64)__umul64hi(all, (r >> 40) << 40); };  // floor(mass * r24 / 2^24)
+  u64 target, base;
+  int grp;
+  if (ngrp <= 64) {  // one wave holds them (up to 32768 logits): no more barriers
+    if (wv != 0) return;
+    const u64 own = lane < ngrp ? mass_bin[lane] : 0;
+    u64 incl = own;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if (before <= target && target < before + m4[q]) {
-      found_bin = 4 * tid + q;
-      found_above = before;
+    for (int o = 1; o < 64; o <<= 1) {
+      const u64 y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
     }
-    before += m4[q];
-  }
-  __syncthreads();
-  if (wv != 0) return;
-  int64_t pick = amax;
-  if (found_bin >= 0) {
-    u64 base = found_above;
-    for (int64_t c = 0; c < per; ++c) {
-      const int64_t blk = (int64_t)found_bin * per + c;
-      const u32x4 q = block_piece(blk);
-      u64 s8 = 0;
+    target = target_of(__shfl(incl, 63, 64));
+    const uint64_t in = __ballot(incl - own <= target && target < incl);
+    grp = in ? __builtin_ctzll(in) : -1;
+    base = __shfl(incl - own, max(grp, 0), 64);
+  } else {
+    // groups 4 tid .. + 3 of this thread; prefix = all - suffix
+    u64 own = 0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s8 += kept_mass(q, e);
+    for (int q = 0; q < 4; ++q) {
+      m4[q] = 4 * tid + q < ngrp ? mass_bin[4 * tid + q] : 0;
+      own += m4[q];
+    }
+    const u64 suffix = block_suffix<u64>(own, sh64);
+    __syncthreads();
+    if (tid == 0) {
+      found_above = suffix;  // the whole mass
+      found_bin = -1;
+    }
+    __syncthreads();
+    u64 before = found_above - suffix;
+    target = target_of(found_above);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (before <= target && target < before + m4[q]) {
+        found_bin = 4 * tid + q;
+        found_above = before;
+      }
+      before += m4[q];
+    }
+    __syncthreads();
+    if (wv != 0) return;
+    grp = found_bin;
+    base = found_above;
+  }
+  int64_t pick = amax;
+  if (grp >= 0) {
+    for (int64_t c = 0; c < per; ++c) {
+      const int64_t blk = (int64_t)grp * per + c;
+      const u32x4 q = block_piece(blk);
+      u64 m8[8], s8 = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        m8[e] = kept_mass(q, e);
+        s8 += m8[e];
+      }
       u64 incl = s8;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -4199,9 +4247,8 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
         int64_t hit = amax;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const u64 m = kept_mass(q, e);
-          if (at <= target && target < at + m) hit = blk * 512 + 8 * lane + e;
-          at += m;
+          if (at <= target && target < at + m8[e]) hit = blk * 512 + 8 * lane + e;
+          at += m8[e];
         }
         pick = hit;
       }

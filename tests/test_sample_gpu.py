@@ -160,7 +160,7 @@ def _expected_draw(row, T, k, p, seed, r):
 
 
 @pytest.mark.parametrize("vocab,std", [(128256, 2.0), (128256, 0.01), (5000, 3.0), (1001, 2.0), (517, 40.0), (9, 1.0),
-                                       (300000, 2.0), (2200000, 2.0)])
+                                       (32768, 2.0), (32769, 2.0), (300000, 2.0), (2200000, 2.0)])
 @pytest.mark.parametrize("k,p", [(0, 1.0), (50, 1.0), (0, 0.9), (50, 0.9), (1000, 0.3), (3, 0.0), (0, 0.999)])
 def test_draw_follows_the_rule(dev, vocab, std, k, p):
     """Every threshold combination against the rule in float64: rows aligned
@@ -177,6 +177,21 @@ def test_draw_follows_the_rule(dev, vocab, std, k, p):
     for r in range(n):
         _, near = _expected_draw(lg[r], T, k, p, 21, r)
         assert got[r] in near, (r, got[r], near)
+
+
+@pytest.mark.parametrize("vocab", [9, 511, 1003, 32769])
+@pytest.mark.parametrize("at", [0, -1])
+def test_draw_without_thresholds_sees_a_nan_anywhere(dev, vocab, at):
+    """A NaN below every value (0xffff, the bits that stand for logits past
+    the row) as the first or last logit of a row that is not whole pieces."""
+    lg = torch.randn(2, vocab, generator=torch.Generator().manual_seed(vocab)).to(torch.bfloat16)
+    top = lg[1, 1:-1].float().argmax().item() + 1
+    lg[1, at] = torch.tensor([-1], dtype=torch.int16).view(torch.bfloat16)[0]
+    lg[1, top] += 1
+    for seed in range(6):
+        got = _run(lg.to(dev), True, temperature=50.0, seed=seed).tolist()
+        assert got[1] == top
+    assert len({_run(lg.to(dev), True, temperature=50.0, seed=s).tolist()[0] for s in range(6)}) > 1
 
 
 def test_draw_with_nan_or_inf_is_the_largest(dev):
