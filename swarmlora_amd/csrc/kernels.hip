@@ -5017,13 +5017,15 @@ int launch_prefill_gemm(TiledArgs a, const PrefillPlan& p, hipStream_t st) {
 // 28672 x 8192 97 / 124 / 142 -> 71 / 72 / 76; 28672 x 4096 50 / 61 / 75 -> 38
 // / 39 / 42; 36864 x 4096 (a second workgroup on every eighth CU) 62 / 78 / 94
 // -> 60 / 63 / 71.
-// Where the line lies: 9/16 of a tile a CU for any rows (18944 x 3584, 0.58:
-// 37 / 46 / 60 -> 32 / 33 / 37; 16384 x 4096, 0.50, one row 31.4 -> 33.1), 7/16
-// above 16 rows, where the partials weigh more (14336 x 4096, 0.44, 28 rows
-// 35.4 -> 33.7, 16 rows 31.7 -> 32.9; 11008 x 2048, 0.34, 28 rows 17.7 -> 19.7).
+// Where the line lies, in tiles a CU (times against the sliced kernel, K 2048
+// to 8192): 9/16 for any rows (0.562: 1 row 0.87-1.00, 16 rows 0.79-0.89; 0.50,
+// 16384 x 4096, one row 31.4 -> 33.1 us), 15/32 above 16 rows, where the
+// partials weigh more (0.469: 17 rows 0.88-1.00), 7/16 above 28 (0.438: 17 rows
+// 0.93-1.08, 28 rows 0.87-1.01, 48 rows 0.81-0.94; 0.34, 11008 x 2048, 28 rows
+// 17.7 -> 19.7 us).
 bool wide_gemm_fits(int64_t m, int64_t n, int64_t k) {
   if (m > kSkinnyMaxTok || k % PG_K != 0 || prefill_uses_tiled(k)) return false;
-  return 16 * ((n + 127) / 128) >= (m > 16 ? 7 : 9) * (int64_t)cu_count();
+  return 32 * ((n + 127) / 128) >= (m > 28 ? 14 : m > 16 ? 15 : 18) * (int64_t)cu_count();
 }
 int launch_wide_gemm(TiledArgs a, hipStream_t st) {
   a.n_split = 1;

@@ -156,7 +156,8 @@ def test_a_prompt_gives_the_same_bits_wherever_it_is_in_the_round(dev, rows, n, 
 
 @pytest.mark.parametrize("m,n,k,bias", [
     (16, 18440, 128, True),    # ragged last tile of 128 columns, two stages
-    (17, 14337, 64, False),    # odd row stride, one stage (fewer than the slots)
+    (17, 14337, 64, False),    # odd row stride (below the line of 17 rows)
+    (17, 15361, 64, False),    # ... past it, one stage (fewer than the slots)
     (32, 14336, 192, False),   # a full 32-row tile
     (33, 14340, 320, True),    # the 64-row tile, one valid row past 32
     (64, 28672, 256, False),   # tiles starting at each of four stages
