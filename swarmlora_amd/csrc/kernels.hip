@@ -6608,8 +6608,8 @@ extern "C" int swl_rmsnorm_bf16(const void* x, const void* weight, float eps, vo
 
 extern "C" int swl_silu_mul_bf16(const void* gu, void* out, int64_t n, int64_t inter, void* stream) {
   SWL_CHECK(n >= 0, SWL_ERR_INVALID, "swl_silu_mul_bf16: bad row count");
-  SWL_CHECK(inter > 0 && inter % 8 == 0, SWL_ERR_INVALID, "swl_silu_mul_bf16: inter must be a multiple of 8");
   if (n == 0) return SWL_OK;
+  SWL_CHECK(inter > 0 && inter % 8 == 0, SWL_ERR_INVALID, "swl_silu_mul_bf16: inter must be a multiple of 8");
   SWL_CHECK(gu && out, SWL_ERR_INVALID, "swl_silu_mul_bf16: null argument");
   const dim3 grid((unsigned)(((inter >> 3) + 255) / 256), (unsigned)std::min<int64_t>(n, 65535));
   hipLaunchKernelGGL(silu_mul_dense_kernel, grid, dim3(256), 0, (hipStream_t)stream,

@@ -243,3 +243,4 @@ def test_dense_act_more_rows_than_the_grid(dev):
         torch.cuda.synchronize()
         assert bits_equal(got[c], want)
     assert ops.rms_norm(gu[:0], torch.ones(16, dtype=BF16, device=dev), 1e-5).shape == (0, 16)
+    assert ops.silu_mul(gu[:0], 8).shape == (0, 8) and ops.silu_mul(torch.zeros(0, 24, dtype=BF16, device=dev), 12).shape == (0, 12)
