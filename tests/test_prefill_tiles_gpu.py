@@ -51,6 +51,8 @@ def _round(dev, rows, n, k, cols, ranks, bias=False, seed=0):
     ([70], 130, 2048, [130], [12], False),                           # ... rank not a multiple of 8, n % 4
     ([300, 1, 1, 1], 2048, 1024, [2048], [16, 8, 0, 64], False),
     ([66, 62], 1000, 4160, [1000], [0, 0], True),                    # no adapters: no splits
+    ([1000, 60], 14336, 512, [7168, 7168], [16, 8], True),           # 1024 rows in large tiles, 36 behind
+    ([700, 80, 1], 16400, 512, [8200, 8200], [16, 0, 12], True),     # ... and the delta in both epilogues
 ])
 def test_short_prefill_rounds(dev, rows, n, k, cols, ranks, bias):
     got, want = _round(dev, rows, n, k, cols, ranks, bias)
