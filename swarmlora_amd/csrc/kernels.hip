@@ -3065,12 +3065,6 @@ __global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, in
     __builtin_amdgcn_wave_barrier();  // (LDS accesses of a wave stay in order: the reads precede the next writes)
   }
 
-  // the row sums over the four lane groups
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    l[e] += __shfl_xor(l[e], 16, 64);
-    l[e] += __shfl_xor(l[e], 32, 64);
-  }
   // Sums that are not finite, or of 2^100 and more: an infinity or NaN in V is
   // a NaN in every row of the block (0 times it, in the rows that do not see
   // its key; in the others the probability's two halves, one of them 0 or
@@ -3086,7 +3080,11 @@ __global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, in
     for (int d = 0; d < 8; ++d)
 #pragma unroll
       for (int q = 0; q < 4; ++q) top = max(top, __float_as_uint(acc[e][d][q]) & 0x7fffffffu);
-    bad |= top >= 0x71800000u && l[e] == l[e];  // 2^100
+    // rows whose sum of probabilities is a NaN in one of the four lane groups
+    uint64_t none = __ballot(l[e] != l[e]);
+    none |= none >> 32;
+    none |= none >> 16;
+    bad |= top >= 0x71800000u && !((uint32_t)none >> col & 1);  // 2^100
   }
   const bool any_bad = __ballot(bad) != 0;
   if (lane == 0) vbad[kh] = any_bad ? 1 : 0;
@@ -3099,8 +3097,13 @@ __global__ __launch_bounds__(64 * KH, 2) void attn_prefill_kernel(AttnArgs a, in
     return;
   }
 
-  // the KH waves of a row merged pairwise through LDS (each lane meets the
-  // same lane of the other wave)
+  // the row sums over the four lane groups, then the KH waves of a row merged
+  // pairwise through LDS (each lane meets the same lane of the other wave)
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    l[e] += __shfl_xor(l[e], 16, 64);
+    l[e] += __shfl_xor(l[e], 32, 64);
+  }
   for (int half = KH / 2; half >= 1; half >>= 1) {
     if (half < KH / 2) __syncthreads();
     float* mg = reinterpret_cast<float*>(pa_lds) + (int64_t)(kh % half) * 68 * 64;
