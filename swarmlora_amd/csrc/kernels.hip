@@ -22,7 +22,8 @@
 //                           128x128 for short rounds) MFMA tiles fed by
 //                           LDS-DMA, rows read in place from the slot buffers,
 //                           the LoRA delta as extra k-steps; 128 columns by 32
-//                           or 64 rows for a row-major LM head.
+//                           or 64 rows for wide row-major products of up to
+//                           64 rows (an LM head).
 //   tiled_kernel            the prefill projection for K not a multiple of 64:
 //                           128x128x64 LDS-staged MFMA tiles over a gathered
 //                           copy, fp32 accumulation, same epilogue.
@@ -2757,8 +2758,9 @@ __global__ __launch_bounds__(128) void rope_append_kernel(AttnArgs a) {
 // the current ones leave their registers.  The probabilities enter as the sum
 // of two bf16 (the rounded value and what the rounding left, 2^-17 of it
 // unaccounted), two products per tile: the result differs from fp32
-// probabilities by far less than its own rounding (measured against 64 bits:
-// 2.5e-3 before and after).
+// probabilities by far less than its own rounding (error against 64 bits over
+// 1 to 1024 tokens and contexts to 3000: 1.60e-3 to 2.09e-3, the same to seven
+// decimals as with fp32 probabilities, shape by shape).
 //
 // What bounded the kernel this replaces was vector work: one query token per
 // workgroup, every K and V row read again for each.  What bounds this one is

@@ -532,7 +532,12 @@ def lora_delta(x: torch.Tensor, a: torch.Tensor, a_kmajor: bool, blocks, rank: i
     if out is None:
         out = torch.empty((m, blocks.total), dtype=BF16, device=x.device)
     # K-slices of the shrink: about 96 workgroups of 32 rows x 64 columns of
-    # A, each with at least 16 k-steps of 32 for its 8 waves
+    # A, each with at least 16 k-steps of 32 for its 8 waves.  Both launches,
+    # us, by workgroups of the shrink: 512 rows of fused QKV (rank 16) 16: 20.8,
+    # 48: 13.2, 96: 12.5, 192: 13.0, 512: 19.7 (the expand reads every slice);
+    # of Down (K 14336) 16: 41.8, 96: 12.9, 256: 10.5; 64 rows of QKV 16: 8.9
+    # (8 slices), 64: 10.6; 1024 rows of Down 96: 21.3, 256: 14.6, so more would
+    # pay where K is long
     n_ks = max(1, min(16, 96 // max(1, -(-m // 32) * -(-nr // 64)), k // 512))
     part = torch.empty(n_ks * m * nr, dtype=torch.float32, device=x.device)
     v = (ctypes.c_int64 * (4 * n))(*blocks.vals)
